@@ -1152,6 +1152,9 @@ int gp_ensemble_create(const gp_params *params, int n, int dtype, gp_ensemble **
     }
     m->member[i]->stream = m->stream;
   }
+  // the power-of-two build steps an ensemble whose members all allow it
+  m->pow2 = 1;
+  for (int i = 0; i < n; i++) m->pow2 = m->pow2 && m->member[i]->pow2;
   *out = e;
   return GP_OK;
 }
