@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
+
 #include "gpstep.h"
 
 #define GP_GRAPH_SLOTS 6
@@ -82,6 +84,8 @@ struct gp_ctx {
   long path_steps[GP_NPATHS];  // steps run per kernel path since the last gp_path_steps reset
   int shape;             // tile shape of the sparse two-pass path (index into the candidate list)
   int shape_set;         // tile shape the tile set was built for (-1: none)
+  double *stage;        // gp_set_state / gp_get_state: fields in transit (on first use), held under stage_mu
+  std::mutex stage_mu;
 };
 
 #define GP_GRAPH_STEPS 32

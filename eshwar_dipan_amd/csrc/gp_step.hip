@@ -237,6 +237,19 @@ static int store_state(gp_ctx *c, S *dphi_dst, S *dmu_dst) {
   return GP_OK;
 }
 
+// The context's buffer for fields in transit from and to host memory (P + C
+// unpadded binary64 planes), allocated on first use and freed with the context;
+// the caller holds stage_mu until its work on it has finished.  Allocating and
+// freeing it on each call cost more than the copies of a small grid.
+static double *staging(gp_ctx *c) {
+  const size_t n = (size_t)c->hp.mesh_x * c->hp.mesh_y;
+  if (!c->stage && hipMalloc((void **)&c->stage, sizeof(double) * n * (c->P + c->C)) != hipSuccess) {
+    (void)hipGetLastError();
+    c->stage = nullptr;
+  }
+  return c->stage;
+}
+
 extern "C" {
 
 const char *gp_strerror(int code) {
@@ -325,6 +338,7 @@ static void free_ctx(gp_ctx *c) {
     if (c->mulo[i]) (void)hipFree(c->mulo[i]);
   }
   if (c->dphi) (void)hipFree(c->dphi);
+  if (c->stage) (void)hipFree(c->stage);
   if (c->dcode) (void)hipFree(c->dcode);
   if (c->dsplit) (void)hipFree(c->dsplit);
   if (c->dcells) (void)hipFree(c->dcells);
@@ -515,8 +529,9 @@ int gp_set_path(gp_ctx *c, int path) {
 int gp_set_state(gp_ctx *c, const double *phi, const double *mu) {
   if (!c || !phi || !mu) return GP_E_ARG;
   size_t n = (size_t)c->hp.mesh_x * c->hp.mesh_y;
-  double *d = nullptr;
-  if (hipMalloc((void **)&d, sizeof(double) * n * (c->P + c->C)) != hipSuccess) return GP_E_NOMEM;
+  std::lock_guard<std::mutex> hold(c->stage_mu);
+  double *d = staging(c);
+  if (!d) return GP_E_NOMEM;
   int rc = GP_OK;
   if (hipMemcpyAsync(d, phi, sizeof(double) * n * c->P, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
       hipMemcpyAsync(d + n * c->P, mu, sizeof(double) * n * c->C, hipMemcpyHostToDevice, c->stream) != hipSuccess)
@@ -524,21 +539,20 @@ int gp_set_state(gp_ctx *c, const double *phi, const double *mu) {
   if (!rc) rc = c->dtype == GP_F64 ? load_state<double, double>(c, d, d + n * c->P) : load_state<float, double>(c, d, d + n * c->P);
   if (!rc && c->dcomp) rc = comp_init(c);
   if (hipStreamSynchronize(c->stream) != hipSuccess && !rc) rc = GP_E_HIP;
-  (void)hipFree(d);
   return rc;
 }
 
 int gp_get_state(gp_ctx *c, double *phi, double *mu) {
   if (!c || !phi || !mu) return GP_E_ARG;
   size_t n = (size_t)c->hp.mesh_x * c->hp.mesh_y;
-  double *d = nullptr;
-  if (hipMalloc((void **)&d, sizeof(double) * n * (c->P + c->C)) != hipSuccess) return GP_E_NOMEM;
+  std::lock_guard<std::mutex> hold(c->stage_mu);
+  double *d = staging(c);
+  if (!d) return GP_E_NOMEM;
   int rc = c->dtype == GP_F64 ? store_state<double, double>(c, d, d + n * c->P) : store_state<float, double>(c, d, d + n * c->P);
   if (!rc && (hipMemcpyAsync(phi, d, sizeof(double) * n * c->P, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
               hipMemcpyAsync(mu, d + n * c->P, sizeof(double) * n * c->C, hipMemcpyDeviceToHost, c->stream) != hipSuccess))
     rc = GP_E_HIP;
   if (hipStreamSynchronize(c->stream) != hipSuccess && !rc) rc = GP_E_HIP;
-  (void)hipFree(d);
   return rc;
 }
 
