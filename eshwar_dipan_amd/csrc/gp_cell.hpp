@@ -83,6 +83,54 @@ struct DevParams {
   unsigned long long lcg_step[2];        // the map of one step's (rows_x-2)(rows_y-2) draws
 };
 
+// The parameters of K of the phases under local indices 0..K-1: the cell
+// functions below take DevParams or this view of it, in which table [a][b] is
+// the full table at [id[a]][id[b]].  The indices are per lane, so the entries
+// come through vector loads (a few KB, resident in L1) where DevParams' come
+// through scalar ones.  id is an array beside the view, not in it: a view that
+// held its own address would stay in scratch.
+template <class T>
+struct SubRow {
+  const T* t;
+  const int* id;
+  __device__ __forceinline__ const T& operator[](int a) const { return t[id[a]]; }
+};
+template <class T>
+struct SubTab {
+  const T (*t)[PM];
+  const int* id;
+  __device__ __forceinline__ SubRow<T> operator[](int a) const { return SubRow<T>{t[id[a]], id}; }
+};
+template <class T>
+struct SubCube {
+  const T (*t)[PM][PM];
+  const int* id;
+  __device__ __forceinline__ SubTab<T> operator[](int a) const { return SubTab<T>{t[id[a]], id}; }
+};
+
+template <class R, int K>
+struct SubParams {
+  const int &obstacle, &anisotropy, &mu_solver, &pair_sym, &pow2_dx, &pow2_dy, &mpi, &mpi_noise;
+  const R &dx, &dy, &dt, &two_dy, &inv_dx, &inv_dy, &inv_two_dy, &epsilon, &inv_eps, &tau, &w_pref, &jscale, &well_at,
+      &Teq, &tgv, &V;
+  SubTab<R> gamma, tau_ab, dab;
+  SubCube<R> gamma_abc;
+  SubTab<R[2][2]> rot, rot_inv;
+  SubRow<R[CM]> at_coef, Bsh, B, Beq, dBbdT, dC, ceqL, ceqS;
+  SubRow<R[CM][CM]> A, cmu;
+  SubRow<R[CM][CM][CM]> dcm;
+  SubRow<R> Cf, dTs, dTl;
+  __device__ __forceinline__ SubParams(const DevParams<R>& f, const int (&id)[K])
+      : obstacle(f.obstacle), anisotropy(f.anisotropy), mu_solver(f.mu_solver), pair_sym(f.pair_sym),
+        pow2_dx(f.pow2_dx), pow2_dy(f.pow2_dy), mpi(f.mpi), mpi_noise(f.mpi_noise), dx(f.dx), dy(f.dy), dt(f.dt),
+        two_dy(f.two_dy), inv_dx(f.inv_dx), inv_dy(f.inv_dy), inv_two_dy(f.inv_two_dy), epsilon(f.epsilon),
+        inv_eps(f.inv_eps), tau(f.tau), w_pref(f.w_pref), jscale(f.jscale), well_at(f.well_at), Teq(f.Teq),
+        tgv(f.tgv), V(f.V), gamma{f.gamma, id}, tau_ab{f.tau_ab, id}, dab{f.dab, id}, gamma_abc{f.gamma_abc, id},
+        rot{f.rot, id}, rot_inv{f.rot_inv, id}, at_coef{f.at_coef, id}, Bsh{f.Bsh, id}, B{f.B, id}, Beq{f.Beq, id},
+        dBbdT{f.dBbdT, id}, dC{f.dC, id}, ceqL{f.ceqL, id}, ceqS{f.ceqS, id}, A{f.A, id}, cmu{f.cmu, id},
+        dcm{f.dcm, id}, Cf{f.Cf, id}, dTs{f.dTs, id}, dTl{f.dTl, id} {}
+};
+
 // drand48's generator: x' = (0x5DEECE66D x + 0xB) mod 2^48, value x' 2^-48
 // (POSIX; glibc's erand48_r builds the double from the 48 bits, so the value is
 // exact).
@@ -114,24 +162,24 @@ struct Ops<float> {
 // Division by a grid spacing.  When the spacing is a power of two, v/d and
 // v*(1/d) round the same real number, so the multiplication is exact; the
 // binary64 path divides otherwise.
-template <class R>
-__device__ __forceinline__ R div_dx(R v, const DevParams<R>& p) {
+template <class R, class Pm>
+__device__ __forceinline__ R div_dx(R v, const Pm& p) {
   #ifdef GP_POW2
   return v * p.inv_dx;
 #else
   if constexpr (Ops<R>::Exact) return p.pow2_dx ? v * p.inv_dx : v / p.dx; else return v * p.inv_dx;
 #endif
 }
-template <class R>
-__device__ __forceinline__ R div_dy(R v, const DevParams<R>& p) {
+template <class R, class Pm>
+__device__ __forceinline__ R div_dy(R v, const Pm& p) {
   #ifdef GP_POW2
   return v * p.inv_dy;
 #else
   if constexpr (Ops<R>::Exact) return p.pow2_dy ? v * p.inv_dy : v / p.dy; else return v * p.inv_dy;
 #endif
 }
-template <class R>
-__device__ __forceinline__ R div_2dy(R v, const DevParams<R>& p) {
+template <class R, class Pm>
+__device__ __forceinline__ R div_2dy(R v, const Pm& p) {
   #ifdef GP_POW2
   return v * p.inv_two_dy;
 #else
@@ -148,8 +196,8 @@ __device__ __forceinline__ R sqrt_nz(R v) {
 // ---------------------------------------------------------------- thermodynamics
 
 // c_a,i(mu)  (functionF_01.h:30-37)
-template <int C, class R>
-__device__ __forceinline__ R c_mu(const DevParams<R>& p, const R* mu, int a, int i) {
+template <int C, class R, class Pm>
+__device__ __forceinline__ R c_mu(const Pm& p, const R* mu, int a, int i) {
   R s = R(0);
 #pragma unroll
   for (int k = 0; k < C; k++) s += p.cmu[a][i][k] * (mu[k] - p.Bsh[a][k]);
@@ -157,8 +205,8 @@ __device__ __forceinline__ R c_mu(const DevParams<R>& p, const R* mu, int a, int
 }
 
 // Mu_a,i(c)  (functionF_01.h:19-29)
-template <int C, class R>
-__device__ __forceinline__ R Mu_of_c(const DevParams<R>& p, const R* c, int a, int i) {
+template <int C, class R, class Pm>
+__device__ __forceinline__ R Mu_of_c(const Pm& p, const R* c, int a, int i) {
   R s = R(2.0) * p.A[a][i][i] * c[i] + p.Bsh[a][i];
 #pragma unroll
   for (int j = 0; j < C; j++)
@@ -167,8 +215,8 @@ __device__ __forceinline__ R Mu_of_c(const DevParams<R>& p, const R* c, int a, i
 }
 
 // f_a(c)  (functionF_01.h:5-18)
-template <int C, class R>
-__device__ __forceinline__ R free_energy(const DevParams<R>& p, const R* c, int a) {
+template <int C, class R, class Pm>
+__device__ __forceinline__ R free_energy(const Pm& p, const R* c, int a) {
   R s = R(0);
 #pragma unroll
   for (int i = 0; i < C; i++) {
@@ -216,8 +264,8 @@ __device__ __forceinline__ R dhphi(const R* ph, int b, int a) {
 }
 
 // psi_b(mu) = f_b(c_b(mu)) - mu.c_b(mu)  (functionF_01.h:41-57, the b-term of dpsi)
-template <int C, class R>
-__device__ __forceinline__ R psi_of_mu(const DevParams<R>& p, const R* mu, int b) {
+template <int C, class R, class Pm>
+__device__ __forceinline__ R psi_of_mu(const Pm& p, const R* mu, int b) {
   R c[C];
   R psi = R(0);
 #pragma unroll
@@ -230,8 +278,8 @@ __device__ __forceinline__ R psi_of_mu(const DevParams<R>& p, const R* mu, int b
 }
 
 // tau(phi)  (functionTau.h:1-16)
-template <int P, class R>
-__device__ __forceinline__ R tau_phi(const DevParams<R>& p, const R* ph) {
+template <int P, class R, class Pm>
+__device__ __forceinline__ R tau_phi(const Pm& p, const R* ph) {
   R s = R(0), s1 = R(0);
 #pragma unroll
   for (int a = 0; a < P; a++)
@@ -267,21 +315,21 @@ __device__ __forceinline__ R temp_row(const DevParams<R>& p, R tb, int y, bool p
 }
 
 // Beq + dBbdT (T - Teq) of c_a(mu) and Mu_a(c) at temperature T (functionF_01.h:19-37)
-template <class R>
-__device__ __forceinline__ R bsh_t(const DevParams<R>& p, int a, int k, R T) {
+template <class R, class Pm>
+__device__ __forceinline__ R bsh_t(const Pm& p, int a, int k, R T) {
   return p.Beq[a][k] + p.dBbdT[a][k] * (T - p.Teq);
 }
 
-template <int C, class R>
-__device__ __forceinline__ R c_mu_t(const DevParams<R>& p, const R* mu, int a, int i, R T) {
+template <int C, class R, class Pm>
+__device__ __forceinline__ R c_mu_t(const Pm& p, const R* mu, int a, int i, R T) {
   R s = R(0);
 #pragma unroll
   for (int k = 0; k < C; k++) s += p.cmu[a][i][k] * (mu[k] - bsh_t(p, a, k, T));
   return s;
 }
 
-template <int C, class R>
-__device__ __forceinline__ R Mu_of_c_t(const DevParams<R>& p, const R* c, int a, int i, R T) {
+template <int C, class R, class Pm>
+__device__ __forceinline__ R Mu_of_c_t(const Pm& p, const R* c, int a, int i, R T) {
   R s = R(2.0) * p.A[a][i][i] * c[i] + bsh_t(p, a, i, T);
 #pragma unroll
   for (int j = 0; j < C; j++)
@@ -291,8 +339,8 @@ __device__ __forceinline__ R Mu_of_c_t(const DevParams<R>& p, const R* c, int a,
 
 // B_a,i(T) and C_a(T) (functionF_01.h:62-104), the tables init_propertymatrices(T)
 // leaves for the phase-field terms of a cell of temperature T
-template <int C, class R>
-__device__ __forceinline__ R B_of_T(const DevParams<R>& p, int L, R T, int i, int a) {
+template <int C, class R, class Pm>
+__device__ __forceinline__ R B_of_T(const Pm& p, int L, R T, int i, int a) {
   if (a == L) return R(0);
   R cl[C], cs[C], sum_c = R(0);
 #pragma unroll
@@ -304,8 +352,8 @@ __device__ __forceinline__ R B_of_T(const DevParams<R>& p, int L, R T, int i, in
   return (R(2.0) * (p.A[L][i][i] * cl[i] - p.A[a][i][i] * cs[i]) + sum_c);
 }
 
-template <int C, class R>
-__device__ __forceinline__ R C_of_T(const DevParams<R>& p, int L, R T, int a) {
+template <int C, class R, class Pm>
+__device__ __forceinline__ R C_of_T(const Pm& p, int L, R T, int a) {
   if (a == L) return R(0);
   R cl[C], cs[C], sum_c = R(0);
 #pragma unroll
@@ -321,8 +369,8 @@ __device__ __forceinline__ R C_of_T(const DevParams<R>& p, int L, R T, int a) {
   return sum_c;
 }
 
-template <int P, int C, class R>
-__device__ __forceinline__ R psi_of_mu_t(const DevParams<R>& p, const R* mu, int b, R T) {
+template <int P, int C, class R, class Pm>
+__device__ __forceinline__ R psi_of_mu_t(const Pm& p, const R* mu, int b, R T) {
   R c[C];
   R psi = R(0);
 #pragma unroll
@@ -345,18 +393,18 @@ __device__ __forceinline__ R psi_of_mu_t(const DevParams<R>& p, const R* mu, int
 }
 
 // the same functions at the run's temperature (tables) or, with NI, at T
-template <int C, bool NI, class R>
-__device__ __forceinline__ R c_mu_(const DevParams<R>& p, const R* mu, int a, int i, R T) {
+template <int C, bool NI, class R, class Pm>
+__device__ __forceinline__ R c_mu_(const Pm& p, const R* mu, int a, int i, R T) {
   if constexpr (NI) return c_mu_t<C>(p, mu, a, i, T);
   else return c_mu<C>(p, mu, a, i);
 }
-template <int C, bool NI, class R>
-__device__ __forceinline__ R Mu_of_c_(const DevParams<R>& p, const R* c, int a, int i, R T) {
+template <int C, bool NI, class R, class Pm>
+__device__ __forceinline__ R Mu_of_c_(const Pm& p, const R* c, int a, int i, R T) {
   if constexpr (NI) return Mu_of_c_t<C>(p, c, a, i, T);
   else return Mu_of_c<C>(p, c, a, i);
 }
-template <int P, int C, bool NI, class R>
-__device__ __forceinline__ R psi_of_mu_(const DevParams<R>& p, const R* mu, int b, R T) {
+template <int P, int C, bool NI, class R, class Pm>
+__device__ __forceinline__ R psi_of_mu_(const Pm& p, const R* mu, int b, R T) {
   if constexpr (NI) return psi_of_mu_t<P, C>(p, mu, b, T);
   else return psi_of_mu<C>(p, mu, b);
 }
@@ -427,8 +475,8 @@ struct Nbhd {
   bool present[P];         // phase b is nonzero somewhere in the 3x3 block
 };
 
-template <int P, class R>
-__device__ __forceinline__ void make_nbhd(const DevParams<R>& p, const R (&v)[P][3][3], Nbhd<P, R>& n) {
+template <int P, class R, class Pm>
+__device__ __forceinline__ void make_nbhd(const Pm& p, const R (&v)[P][3][3], Nbhd<P, R>& n) {
 #pragma unroll
   for (int a = 0; a < P; a++) {
     bool nz = false;
@@ -460,8 +508,8 @@ __device__ __forceinline__ void make_nbhd(const DevParams<R>& p, const R (&v)[P]
 // ---------------------------------------------------------------- delta-phi
 
 // dA/dphi_a  (function_A_00.h:4-24 isotropic; function_A_01.h:4-71 anisotropic)
-template <int P, class R>
-__device__ __forceinline__ R dAdphi(const DevParams<R>& p, const Nbhd<P, R>& n, int a) {
+template <int P, class R, class Pm>
+__device__ __forceinline__ R dAdphi(const Pm& p, const Nbhd<P, R>& n, int a) {
   if (!p.anisotropy) {
     R sum = R(0);
 #pragma unroll
@@ -511,8 +559,8 @@ struct FaceQ {
   R rd[2];     // R^-1 * da_c/dq
 };
 
-template <class R>
-__device__ __forceinline__ void face_q(const DevParams<R>& p, int a, int b, R u0, R u1, R flux, FaceQ<R>& f) {
+template <class R, class Pm>
+__device__ __forceinline__ void face_q(const Pm& p, int a, int b, R u0, R u1, R flux, FaceQ<R>& f) {
   R u[2] = {u0, u1}, q[2], d[2];
   rot2(p.rot[a][b], u, q);
   f.flux = flux;
@@ -524,8 +572,8 @@ __device__ __forceinline__ void face_q(const DevParams<R>& p, int a, int b, R u0
 }
 
 // div (dA / d grad phi_a)  (function_A_00.h:25-58 isotropic; function_A_01.h:101-219 anisotropic)
-template <int P, class R>
-__device__ __forceinline__ R divdAdgradphi(const DevParams<R>& p, const Nbhd<P, R>& n, int a) {
+template <int P, class R, class Pm>
+__device__ __forceinline__ R divdAdgradphi(const Pm& p, const Nbhd<P, R>& n, int a) {
   if (!p.anisotropy) {
     R sum = R(0);
 #pragma unroll
@@ -584,8 +632,8 @@ __device__ __forceinline__ R divdAdgradphi(const DevParams<R>& p, const Nbhd<P, 
 // only in the sign of a zero, which leaves nonzero sums unchanged; the results
 // are returned as dA = 2(s1+s2) (entering lam as -dA + dG, where either zero
 // gives +0) and dG = 2(s1+s2) + 0 (zero normalised as in divdAdgradphi).
-template <int P, class R>
-__device__ __forceinline__ void aniso_pairs(const DevParams<R>& p, const Nbhd<P, R>& n, const bool* want, R* dA,
+template <int P, class R, class Pm>
+__device__ __forceinline__ void aniso_pairs(const Pm& p, const Nbhd<P, R>& n, const bool* want, R* dA,
                                             R* dG) {
   R a1[P], a2[P], g1[P], g2[P];
 #pragma unroll
@@ -675,8 +723,8 @@ __device__ __forceinline__ void aniso_pairs(const DevParams<R>& p, const Nbhd<P,
 }
 
 // dw/dphi_a  (functionW_01.h:6-39 obstacle, functionW_02.h:4-33 well)
-template <int P, class R>
-__device__ __forceinline__ R dwdphi(const DevParams<R>& p, const R* ph, const bool* act, int a) {
+template <int P, class R, class Pm>
+__device__ __forceinline__ R dwdphi(const Pm& p, const R* ph, const bool* act, int a) {
   R sum = R(0);
   if (p.obstacle) {
 #pragma unroll
@@ -749,8 +797,8 @@ __device__ __forceinline__ void project_simplex(const R* ph, const bool* act, R*
 
 // Active phases of a cell: |div phi_a| > 0 (calculate_divergence_phasefield.h:9-16).
 // Returns whether any phase is active.
-template <int P, class R>
-__device__ __forceinline__ bool cell_active(const DevParams<R>& p, const Nbhd<P, R>& n, bool* act) {
+template <int P, class R, class Pm>
+__device__ __forceinline__ bool cell_active(const Pm& p, const Nbhd<P, R>& n, bool* act) {
   bool any = false;
 #pragma unroll
   for (int a = 0; a < P; a++) {
@@ -771,8 +819,8 @@ __device__ __forceinline__ bool cell_active(const DevParams<R>& p, const Nbhd<P,
 // dpsi / V under GP_MPI_DPSI_V, and mnz (4 Amp drand48() of the cell) adds
 // mnz phi_a (1 - phi_a) dpsi / V under p.mpi_noise
 // (MPI calculate_divergence_phasefield.h:335-343).
-template <int P, int C, class R, bool NI = false, bool MPI = false>
-__device__ __forceinline__ void cell_dphi_rest(const DevParams<R>& p, const Nbhd<P, R>& n, const R* mu,
+template <int P, int C, class R, bool NI = false, bool MPI = false, class Pm>
+__device__ __forceinline__ void cell_dphi_rest(const Pm& p, const Nbhd<P, R>& n, const R* mu,
                                                const bool* act, bool any, bool pairs, R* dA, R* dG, R* dp,
                                                R T = R(0), const uint32_t* nzw = nullptr, R amp = R(0),
                                                R mnz = R(0)) {
@@ -818,8 +866,8 @@ __device__ __forceinline__ void cell_dphi_rest(const DevParams<R>& p, const Nbhd
 
 // delta-phi of one cell  (calculate_divergence_phasefield.h:4-62)
 // (T: the cell's temperature, used with NI only)
-template <int P, int C, class R, bool NI = false, bool MPI = false>
-__device__ __forceinline__ void cell_dphi(const DevParams<R>& p, const Nbhd<P, R>& n, const R* mu, R* dp,
+template <int P, int C, class R, bool NI = false, bool MPI = false, class Pm>
+__device__ __forceinline__ void cell_dphi(const Pm& p, const Nbhd<P, R>& n, const R* mu, R* dp,
                                           R T = R(0), const uint32_t* nzw = nullptr, R amp = R(0),
                                           R mnz = R(0)) {
   bool act[P];
@@ -841,8 +889,8 @@ __device__ __forceinline__ R s_phi(const R* ph, int a) {
 }
 
 // D_ij of one cell  (functionD.h:1-15)
-template <int P, int C, class R>
-__device__ __forceinline__ void cell_D(const DevParams<R>& p, const R* ph, R (&D)[C][C]) {
+template <int P, int C, class R, class Pm>
+__device__ __forceinline__ void cell_D(const Pm& p, const R* ph, R (&D)[C][C]) {
 #pragma unroll
   for (int i = 0; i < C; i++)
 #pragma unroll
@@ -861,8 +909,8 @@ __device__ __forceinline__ void cell_D(const DevParams<R>& p, const R* ph, R (&D
 // ct_p / ct_q: tangential centred gradients at p and q (the face's tangential
 // gradient is their mean), phase fields, potentials and delta-phi of both cells.
 // With NI, c(mu) of the two cells is taken at their temperatures T_p, T_q.
-template <int P, int C, class R, bool NI = false>
-__device__ __forceinline__ void face_jat(const DevParams<R>& p, const R* g_p, const R* ct_p, const R* ct_q,
+template <int P, int C, class R, bool NI = false, class Pm>
+__device__ __forceinline__ void face_jat(const Pm& p, const R* g_p, const R* ct_p, const R* ct_q,
                                          const R* ph_p, const R* ph_q, const R* mu_p, const R* mu_q,
                                          const R* dp_p, const R* dp_q, bool enabled, R* jat, R T_p = R(0),
                                          R T_q = R(0)) {
@@ -979,8 +1027,8 @@ __device__ __forceinline__ void lu_inverse(R (&a)[C][C], R (&inv)[C][C]) {
 // (calculate_divergence_concentration.h:4-153).  jat*/Dm*/gm*: antitrapping flux,
 // face mobility and mu gradient on the faces front (x|x+1), back (x-1|x),
 // right (y|y+1), left (y-1|y).
-template <int P, int C, class R, bool NI = false>
-__device__ __forceinline__ void cell_update(const DevParams<R>& p, const R* ph, const R* mu, const R* dp,
+template <int P, int C, class R, bool NI = false, class Pm>
+__device__ __forceinline__ void cell_update(const Pm& p, const R* ph, const R* mu, const R* dp,
                                             const R* jf, const R* jb, const R* jr, const R* jl,
                                             const R (&Dmf)[C][C], const R (&Dmb)[C][C],
                                             const R (&Dmr)[C][C], const R (&Dml)[C][C],
@@ -1126,8 +1174,8 @@ __device__ __forceinline__ void cell_update(const DevParams<R>& p, const R* ph, 
 // sum2 = 0; function_A_00.h returns 2*sum), obstacle/well terms without sign
 // tests (functionW_01.h:41-63, functionW_02.h:35-58), unweighted projection
 // (simplex_projection.h:50-90).
-template <int P, class R>
-__device__ __forceinline__ R dwdphi_smooth(const DevParams<R>& p, const R* ph, const bool* act, int a) {
+template <int P, class R, class Pm>
+__device__ __forceinline__ R dwdphi_smooth(const Pm& p, const R* ph, const bool* act, int a) {
   R sum = R(0);
 #pragma unroll
   for (int b = 0; b < P; b++)
@@ -1172,8 +1220,8 @@ __device__ __forceinline__ void project_unweighted(const R* ph, const bool* act,
   }
 }
 
-template <int P, int C, class R>
-__device__ __forceinline__ void cell_dphi_smooth(const DevParams<R>& p, const Nbhd<P, R>& n, R* dp) {
+template <int P, int C, class R, class Pm>
+__device__ __forceinline__ void cell_dphi_smooth(const Pm& p, const Nbhd<P, R>& n, R* dp) {
   R divphi[P], lam[P];
   bool act[P];
 #pragma unroll
@@ -1223,8 +1271,8 @@ __device__ __forceinline__ void cell_dphi_smooth(const DevParams<R>& p, const Nb
 
 // mu update of the smoothing sweep: diffusion alone, general LU inverse for any
 // solver flag, mu + delta_mu (calculate_divergence_concentration.h:154-253)
-template <int P, int C, class R>
-__device__ __forceinline__ void cell_update_smooth(const DevParams<R>& p, const R* ph, const R* mu,
+template <int P, int C, class R, class Pm>
+__device__ __forceinline__ void cell_update_smooth(const Pm& p, const R* ph, const R* mu,
                                                    const R (&Dmf)[C][C], const R (&Dmb)[C][C],
                                                    const R (&Dmr)[C][C], const R (&Dml)[C][C],
                                                    const R* gmf, const R* gmb, const R* gmr, const R* gml,

@@ -42,16 +42,13 @@ namespace GPK_NS {
 // SIMD leave (the dense phase sweep spilled 2.5 KB per lane, the dense mu
 // sweep 0.6 KB): its dense sweeps run at one wave per SIMD (1.6x the merged
 // launch at two waves).  Binary32 spills 0.8 KB and is faster at two waves.
+// With passes by the phases a cell holds the launches are separate too: merged,
+// the light waves at six phases were held to the dense pass's two per SIMD (64
+// us at 1531 x 1021, against 42 + 21 us for the two launches).
 template <int P, class R>
 constexpr bool onehot_wide() { return P >= 9; }
 template <int P, class R>
 constexpr int onehot_dense_waves() { return onehot_wide<P, R>() && sizeof(R) == 8 ? 1 : GP_WAVES_PER_EU; }
-// The light mu sweep of those split launches in binary64: unbounded it takes 242 registers
-// at nine phases in binary64 (two waves per SIMD); bounded to six waves it
-// spills, but the sweep is faster (4096^2, 9 phases: 1.03e10 -> 1.14e10
-// cell-updates/s for the step; bounds of 3, 4, 5 gave 1.09e10, 1.11e10, 1.13e10).
-template <int P, class R>
-constexpr int onehot_light_waves() { return onehot_wide<P, R>() && sizeof(R) == 8 ? 6 : 1; }
 // The one-hot path's dense mu sweep takes two waves per listed cell (the x and
 // y antitrapping faces side by side) below nine phases, one lane per cell from
 // nine: at 4096^2 and nine phases one lane is 15% (binary64) and 6% (binary32)
@@ -244,13 +241,17 @@ __device__ __forceinline__ int conc_apply(const DevParams<R>& p, const R (&v)[P]
       mulo_o[idx(p, k, x, y)] = lo_n;
     }
   }
-  int a1 = -1, nz = 0;
+  int a1 = -1, n1 = 0, nz = 0;  // the exact one-hot bits
 #pragma unroll
   for (int a = 0; a < P; a++) {
-    if (pho[a] == R(1.0)) a1 = a;
-    else if (pho[a] != R(0)) nz++;
+    if (pho[a] == R(1.0)) {
+      a1 = a;
+      n1++;
+    } else if (pho[a] != R(0) || signbit(pho[a])) {
+      nz++;
+    }
   }
-  return nz == 0 ? a1 : -1;
+  return nz == 0 && n1 == 1 ? a1 : -1;
 }
 
 // mu and phi update of interior cell (x,y) with its ghost images (all four

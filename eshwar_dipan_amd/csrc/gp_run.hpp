@@ -199,7 +199,7 @@ int run_sparse(gp_ctx *c, long nsteps) {
     hipLaunchKernelGGL(k_clear_counts<0>, dim3(1), dim3(64), 0, c->stream, c->dcnt);
     c->cnt_par = c->cur;
     hipLaunchKernelGGL((k_flags<P, R, T::TX, T::TY>), dim3(nt), dim3(256), 0, c->stream, inst, tinst, c->cur,
-                       c->dflag[c->cur]);
+                       c->dflag[c->cur], c->dflag[c->cur ^ 1]);
     c->flags_valid = 1;
   }
   const int g_if = std::min(nt, 2048), g_bulk = std::min(nt, 4096);
