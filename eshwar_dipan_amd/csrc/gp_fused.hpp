@@ -743,7 +743,7 @@ __global__ void __launch_bounds__(256) GP_HEAVY k_conc_cells(const DevParams<R>*
 // appending blocks of a launch spread their device-scope atomics over kSegs
 // addresses instead of queueing on one (such atomics serialise at about 12 ns
 // each per address on MI355X: one per block of a 1024^2 sweep on 8 addresses
-// cost 8 us).  Segment k holds 256 cells per block of its class (the blocks of
+// cost 8 us).  Segment k holds every cell of the blocks of its class (those of
 // a launch with index = k mod kSegs), so it cannot overflow; the counters sit
 // kSegStride ints apart, and a dense lane finds listed cell i by walking the
 // kSegs counts.  kSegs is a multiple of 8, so a segment's blocks share an XCD;
@@ -753,13 +753,29 @@ constexpr int kSegs = 8;
 constexpr int kSegStride = 32;
 constexpr int kSegInts = 2 * kSegs * kSegStride;  // phase-sweep counters, then mu-sweep counters
 
-// First slot of segment k of a list written by a launch of nblk blocks.
+// Cells per block of the light mu sweep and of the light phase sweep (kPhaseCols
+// columns per lane).
+constexpr int kMuCells = BX * BY;
+constexpr int kPhaseCols = 4;
+constexpr int kPhaseCells = BX * BY * kPhaseCols;
+
+// First slot of segment k of a list written by a launch of nblk blocks of
+// `cells` cells.
+template <int cells>
 __host__ __device__ __forceinline__ int seg_base(int k, int nblk) {
   const int q = nblk / kSegs, r = nblk % kSegs;
-  return (k * q + (k < r ? k : r)) * (BX * BY);
+  return (k * q + (k < r ? k : r)) * cells;
 }
 
-// cell_append into segment L mod kSegs (cnt: the list's kSegs counters).
+// Grid of the light phase sweep over [2, rows-3]^2: groups of kPhaseCols
+// columns from column 0 on (a group is one aligned word of the byte planes).
+__host__ __device__ inline dim3 phase_light_grid(int rx, int ry) {
+  return dim3(((ry - 2 + kPhaseCols - 1) / kPhaseCols + BX - 1) / BX, (rx - 4 + BY - 1) / BY);
+}
+
+// cell_append into segment L mod kSegs (cnt: the list's kSegs counters) of a
+// list whose blocks hold `cells` cells each.
+template <int cells>
 __device__ __forceinline__ void cell_append_seg(bool want, int x, int y, int L, int nblk, int* __restrict__ list,
                                                 int* __restrict__ cnt) {
   __shared__ int wn[BY + 1];
@@ -778,18 +794,20 @@ __device__ __forceinline__ void cell_append_seg(bool want, int x, int y, int L, 
     wn[BY] = t ? atomicAdd(cnt + kSegStride * (L % kSegs), t) : 0;
   }
   __syncthreads();
-  if (want) list[seg_base(L % kSegs, nblk) + wn[BY] + wn[w] + __popcll(m & ((1ull << lane) - 1ull))] = (x << 16) | y;
+  if (want)
+    list[seg_base<cells>(L % kSegs, nblk) + wn[BY] + wn[w] + __popcll(m & ((1ull << lane) - 1ull))] = (x << 16) | y;
 }
 
 // Listed cells of a segmented list: n = their number; cell i (< n) is entry
 // seg_at(i) of the list.
+template <int cells>
 struct SegList {
   int c[kSegs], n, nblk;
   __device__ __forceinline__ SegList(const int* __restrict__ cnt, int nblk_) : n(0), nblk(nblk_) {
 #pragma unroll
     for (int k = 0; k < kSegs; k++) {
       const int q = nblk / kSegs, r = nblk % kSegs;
-      c[k] = min(cnt[kSegStride * k], (q + (k < r ? 1 : 0)) * (BX * BY));  // a segment holds at most its capacity
+      c[k] = min(cnt[kSegStride * k], (q + (k < r ? 1 : 0)) * cells);  // a segment holds at most its capacity
       n += c[k];
     }
   }
@@ -801,7 +819,7 @@ struct SegList {
         i -= c[j];
         k = j + 1;
       }
-    return seg_base(k, nblk) + i;
+    return seg_base<cells>(k, nblk) + i;
   }
 };
 
@@ -834,38 +852,120 @@ __global__ void k_clear_seg(int* __restrict__ cnt) {
   for (int i = threadIdx.x; i < kSegInts; i += blockDim.x) cnt[i] = 0;
 }
 
+// phase_uniform, four phases at a time (with the loads of all nine in flight
+// the light phase sweep took 240 registers), a wave leaving when none of its
+// cells can still be uniform; ph is set where the result is true.
+template <int P, class R>
+__device__ __forceinline__ bool phase_uniform_by4(const DevParams<R>& p, const R* __restrict__ phi, int x, int y,
+                                                  R* ph) {
+  bool u = true;
+#pragma unroll 1
+  for (int a0 = 0; a0 < P && u; a0 += 4) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int a = a0 + j;
+      if (P % 4 != 0 && a >= P) break;
+      const R c = phi[idx(p, a, x, y)];
+      const R f = phi[idx(p, a, x + 1, y)], b = phi[idx(p, a, x - 1, y)];
+      const R r = phi[idx(p, a, x, y + 1)], l = phi[idx(p, a, x, y - 1)];
+      u &= (f == c) & (b == c) & (r == c) & (l == c);
+    }
+  }
+  if (u) {
+#pragma unroll
+    for (int a = 0; a < P; a++) ph[a] = phi[idx(p, a, x, y)];
+  }
+  return u;
+}
+
 // Light phase sweep of path 6 over [2, rows-3]^2: k_phase_light with the
 // one-hot shortcut of the current buffer's plane oh, appending to the
 // segmented phase-sweep list (lists + kSegInts, counters lists[0..]).  Clears
 // the mu-sweep counters, which the previous step's dense kernel has finished
 // reading.
+//
+// Almost every cell takes the shortcut, so the sweep is bound by the number of
+// waves and of appends, not by its two bytes per cell: a lane first takes the
+// kPhaseCols columns of one aligned word of the byte planes, and compares the
+// words of the row, of the rows beside it and of the columns beside it.  The
+// block's cells that fail (and those outside [4, mesh + 1]^2, whose cross
+// leaves the interior) are gathered in LDS and looked at one per lane: left to
+// the lane that found them, they ran one after another, and the sweep took 3-4
+// times as long on states with wide interfaces.  One column per lane against
+// this: 8.8 -> 6.3 us at 1024^2 and four phases, 17.6 -> 11.4 us at 1531 x 1021
+// and six, 117 -> 70 us (binary32: 116 -> 63 us) at 4096^2 and nine.
 template <int P, class R>
 __global__ void __launch_bounds__(BX * BY) k_phase_light_oh(const DevParams<R>* __restrict__ prm,
                                                             const R* __restrict__ phi,
                                                             const signed char* __restrict__ oh, R* __restrict__ dphi,
                                                             signed char* __restrict__ code, int* __restrict__ lists) {
+  static_assert(kPhaseCols == 4, "a group is one 32-bit word");
+  __shared__ short todo[kPhaseCells];  // row of the block << 8 | column of the block
+  __shared__ int tn[BY];
   const DevParams<R>& p = *prm;
   int bx, by;
   blk_xy(bx, by);
-  const int y = 2 + bx * BX + threadIdx.x;
-  const int x = 2 + by * BY + threadIdx.y;
+  const int yb = bx * BX * kPhaseCols, xb = 2 + by * BY;
+  const int y0 = yb + threadIdx.x * kPhaseCols, x = xb + threadIdx.y;
   const int L = blockIdx.y * gridDim.x + blockIdx.x, nblk = gridDim.x * gridDim.y;
   if (L == 0 && threadIdx.y == 0 && threadIdx.x < kSegs) lists[kSegs * kSegStride + kSegStride * threadIdx.x] = 0;
-  bool heavy = false;
-  if (x <= p.rx - 3 && y <= p.ry - 3) {
-    const size_t i = (size_t)x * p.pitch + y;
-    int o = -1;
-    if (x >= 4 && x <= p.mesh_x + 1 && y >= 4 && y <= p.mesh_y + 1) {  // the cross lies in the interior
-      o = oh[i];
-      o = oh[i + p.pitch] == o && oh[i - p.pitch] == o && oh[i + 1] == o && oh[i - 1] == o ? o : -1;
+  unsigned left = 0;  // bit j: cell j is looked at
+  if (x <= p.rx - 3 && y0 <= p.ry - 3) {
+    const size_t i = (size_t)x * p.pitch + y0;  // pitch and y0 are multiples of 4
+    unsigned sure = 0, w = 0;                   // bit 8 j + 7: cell j takes the shortcut; the codes
+    if (x >= 4 && x <= p.mesh_x + 1) {
+      w = *(const unsigned*)(oh + i);
+      const unsigned u = *(const unsigned*)(oh + i + p.pitch), d = *(const unsigned*)(oh + i - p.pitch);
+      const unsigned l = y0 ? (unsigned char)oh[i - 1] : 0, r = y0 + 4 < p.pitch ? (unsigned char)oh[i + 4] : 0;
+      const unsigned t = (w ^ u) | (w ^ d) | (w ^ (w << 8 | l)) | (w ^ (w >> 8 | r << 24)) | (w & 0x80808080u);
+      sure = ~(((t & 0x7f7f7f7fu) + 0x7f7f7f7fu) | t) & 0x80808080u;  // bytes of t that are zero
+#pragma unroll
+      for (int j = 0; j < kPhaseCols; j++)
+        if (y0 + j < 4 || y0 + j > p.mesh_y + 1) sure &= ~(0x80u << (8 * j));
     }
-    if (o >= 0) {
-      code[i] = (signed char)o;
+    if (sure == 0x80808080u) {
+      *(unsigned*)(code + i) = w;
     } else {
+#pragma unroll
+      for (int j = 0; j < kPhaseCols; j++) {
+        if (y0 + j < 2 || y0 + j > p.ry - 3) continue;
+        if ((sure >> (8 * j + 7)) & 1) code[i + j] = (signed char)(w >> (8 * j));
+        else left |= 1u << j;
+      }
+    }
+  }
+  // the cells left, in the order of the rows and columns
+  int below = 0, all = 0;
+#pragma unroll
+  for (int j = 0; j < kPhaseCols; j++) {
+    const unsigned long long m = __ballot((left >> j) & 1);
+    below += __popcll(m & ((1ull << threadIdx.x) - 1ull));
+    all += __popcll(m);
+  }
+  if (threadIdx.x == 0) tn[threadIdx.y] = all;
+  __syncthreads();
+  int n = 0;
+#pragma unroll
+  for (int i = 0; i < BY; i++) {
+    if (i < (int)threadIdx.y) below += tn[i];
+    n += tn[i];
+  }
+#pragma unroll
+  for (int j = 0; j < kPhaseCols; j++)
+    if ((left >> j) & 1) todo[below++] = (short)(threadIdx.y << 8 | (threadIdx.x * kPhaseCols + j));
+  __syncthreads();
+  for (int base = 0; base < n; base += BX * BY) {  // the same passes for every lane of the block
+    const int k = base + (int)threadIdx.y * BX + (int)threadIdx.x;
+    bool heavy = false;
+    int cx = 0, cy = 0;
+    if (k < n) {
+      cx = xb + (todo[k] >> 8);
+      cy = yb + (todo[k] & 0xff);
+      signed char* cd_o = code + (size_t)cx * p.pitch + cy;
       R ph[P];
-      if (!phase_uniform<P>(p, phi, x, y, ph)) {  // possibly active: the dense kernel decides
+      if (!phase_uniform_by4<P>(p, phi, cx, cy, ph)) {  // possibly active: the dense kernel decides
         heavy = true;
-        code[i] = -1;
+        *cd_o = -1;
       } else {
         R dp[P];
         bool act[P];
@@ -879,15 +979,15 @@ __global__ void __launch_bounds__(BX * BY) k_phase_light_oh(const DevParams<R>* 
 #pragma unroll
         for (int a = 0; a < P; a++) zero = zero && dp[a] == R(0) && !signbit(dp[a]);
         const int cd = zero ? onehot_bits<P>(ph) : -1;
-        code[i] = (signed char)cd;
+        *cd_o = (signed char)cd;
         if (cd < 0) {
 #pragma unroll
-          for (int a = 0; a < P; a++) dphi[idx(p, a, x, y)] = dp[a];
+          for (int a = 0; a < P; a++) dphi[idx(p, a, cx, cy)] = dp[a];
         }
       }
     }
+    cell_append_seg<kPhaseCells>(heavy, cx, cy, L, nblk, lists + kSegInts, lists);
   }
-  cell_append_seg(heavy, x, y, L, nblk, lists + kSegInts, lists);
 }
 
 // Light mu update of path 6 for one interior cell, in two halves: load()
@@ -962,7 +1062,7 @@ __device__ __forceinline__ void light_mu_block(const DevParams<R>& p, int x, int
   const bool in = x <= p.mesh_x + 2 && y <= p.mesh_y + 2;
   const bool heavy = in && lm.load(p, x, y, mu, mulo, code, oh_o);
   if (in) lm.finish(p, x, y, mulo, phi_o, mu_o, mulo_o, oh_o, tb, tsh);
-  cell_append_seg(heavy, x, y, L, nblk, lc, cnt_c);
+  cell_append_seg<kMuCells>(heavy, x, y, L, nblk, lc, cnt_c);
 }
 
 // Dense phase sweep of path 6 over the segmented phase-sweep list (written by
@@ -974,7 +1074,7 @@ __device__ __forceinline__ void phase_cells_seg(const DevParams<R>& p, const R* 
                                                 const int* __restrict__ lists, int nbp, int first, int stride, R tb,
                                                 int tmode, const NoiseRef& nz) {
   const int* lp = lists + kSegInts;
-  const SegList sl(lists, nbp);
+  const SegList<kPhaseCells> sl(lists, nbp);
   for (int i = first; i < sl.n; i += stride) {
     const int e = lp[sl.seg_at(i)], x = e >> 16, y = e & 0xffff;
     if (x < 2 || x > p.rx - 3 || y < 2 || y > p.ry - 3) continue;  // entries are cells of the phase sweep
@@ -1058,7 +1158,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(onehot
   __shared__ R xch[128][2][C];
   const DevParams<R>& p = *prm;
   const int* lc = lists + kSegInts + capp;
-  const SegList sl(lists + kSegs * kSegStride, nbc);
+  const SegList<kMuCells> sl(lists + kSegs * kSegStride, nbc);
   if (blockIdx.x == 0 && threadIdx.x < kSegs) lists[kSegStride * threadIdx.x] = 0;
   if constexpr (onehot_conc_one_lane<P, R>()) {  // one lane per listed cell
     for (int i = blockIdx.x * 256 + threadIdx.x; i < sl.n; i += gridDim.x * 256) {

@@ -389,11 +389,11 @@ template <int P, int C, class R, bool NI>
 int run_onehot(gp_ctx *c, long nsteps) {
   if (c->rx > 65535 || c->ry > 65535) return GP_E_UNSUPPORTED;  // list entries pack x and y in 16 bits
   const dim3 blk(BX, BY);
-  const dim3 gp = phase_grid(c->rx, c->ry);
+  const dim3 gp = phase_light_grid(c->rx, c->ry);
   const int gx = ((int)c->hp.mesh_y + BX - 1) / BX, gy = ((int)c->hp.mesh_x + BY - 1) / BY;
-  const int nbp = (int)(gp.x * gp.y), nbc = gx * gy, capp = nbp * BX * BY;
+  const int nbp = (int)(gp.x * gp.y), nbc = gx * gy, capp = nbp * kPhaseCells;
   if (!c->dcells6) {
-    GP_HIP_CHECK(hipMalloc((void **)&c->dcells6, sizeof(int) * ((size_t)kSegInts + (size_t)(nbp + nbc) * BX * BY)));
+    GP_HIP_CHECK(hipMalloc((void **)&c->dcells6, sizeof(int) * ((size_t)kSegInts + (size_t)capp + (size_t)nbc * kMuCells)));
     hipLaunchKernelGGL(k_clear_seg<0>, dim3(1), dim3(256), 0, c->stream, c->dcells6);
   }
   if (!c->doh) {
@@ -409,7 +409,7 @@ int run_onehot(gp_ctx *c, long nsteps) {
   }
   // dense blocks of the merged launch (a multiple of 8, so that the light
   // blocks keep the hardware's round-robin over the 8 XCDs) and of k_conc_cells_oh
-  const int nd = std::min((nbp + 7) / 8 * 8, GP_ONEHOT_DENSE);
+  const int nd = std::min((nbp * kPhaseCols + 7) / 8 * 8, GP_ONEHOT_DENSE);
   const int gdense = std::min(nbc, GP_ONEHOT_DENSE);
   for (long t = 0; t < nsteps; t++) {
     const R *phi = (const R *)c->phi[c->cur], *mu = (const R *)c->mu[c->cur], *mulo = (const R *)c->mulo[c->cur];
