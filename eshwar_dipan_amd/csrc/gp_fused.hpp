@@ -752,9 +752,6 @@ __global__ void __launch_bounds__(256) GP_HEAVY k_conc_cells(const DevParams<R>*
 constexpr int kSegs = 8;
 constexpr int kSegStride = 32;
 constexpr int kSegInts = 2 * kSegs * kSegStride;  // phase-sweep counters, then mu-sweep counters
-// Beside the counters, for pass i of a dense sweep (few_k): non-zero if that
-// pass left a cell to the next one (cleared with the counters).
-constexpr int kPhaseLeft = 1, kMuLeft = kSegs * kSegStride + 1;
 
 // Cells per block of the light mu sweep and of the light phase sweep (kPhaseCols
 // columns per lane).
@@ -912,7 +909,6 @@ __global__ void __launch_bounds__(BX * BY) k_phase_light_oh(const DevParams<R>* 
   const int y0 = yb + threadIdx.x * kPhaseCols, x = xb + threadIdx.y;
   const int L = blockIdx.y * gridDim.x + blockIdx.x, nblk = gridDim.x * gridDim.y;
   if (L == 0 && threadIdx.y == 0 && threadIdx.x < kSegs) lists[kSegs * kSegStride + kSegStride * threadIdx.x] = 0;
-  if (L == 0 && threadIdx.y == 0 && threadIdx.x < kFewPasses) lists[kMuLeft + threadIdx.x] = 0;
   unsigned left = 0;  // bit j: cell j is looked at
   if (x <= p.rx - 3 && y0 <= p.ry - 3) {
     const size_t i = (size_t)x * p.pitch + y0;  // pitch and y0 are multiples of 4
@@ -1069,210 +1065,21 @@ __device__ __forceinline__ void light_mu_block(const DevParams<R>& p, int x, int
   cell_append_seg<kMuCells>(heavy, x, y, L, nblk, lc, cnt_c);
 }
 
-// Interface cells by the phases they hold.  With P phases a cell's 3x3 block
-// still holds two or three of them, and an absent phase adds exact zeros to
-// every sum: its activity is false, its delta-phi +0, h and dh/dphi_a of it 0,
-// its mobility and susceptibility terms products with 0.  few_phases therefore
-// gives the cell local indices -- the solids present in ascending order, then
-// the liquid, so every sum keeps the order of its terms -- and the cell
-// functions run with K phases on the view SubParams: the same bits with K K
-// pairs instead of P P, and with registers for K phases (nine phases, binary64,
-// K = 4: 84 B of scratch per lane at two waves per SIMD instead of 1472 B at
-// one).  At 4096^2 and nine phases the dense phase sweep took 386 us, and takes
-// 147 + 63 + 10 us in its three passes; the dense mu sweep 433 us, and 209 + 79
-// + 9 us.  At 1531 x 1021 and six phases the step went from 143 to 133 us.  A
-// cell with more than K - 1 solids, or a value whose products could overflow
-// (an absent phase's 0 * inf would be NaN), is left to the next pass.
-//
-// few_phases: bit set of the solids that are non-zero in the 3x3 block, and
-// the local indices; an index past the solids present repeats a solid and
-// stands for a phase that is zero throughout (used: bit per local index).
-// False if the cell holds more than K - 1 solids.
-template <int P, int K, class R>
-__device__ __forceinline__ bool few_phases(const DevParams<R>& p, const R* __restrict__ phi, int x, int y, int* id,
-                                           unsigned& mask, unsigned& used) {
-  mask = 0;
-#pragma unroll
-  for (int a = 0; a < P - 1; a++) {
-    bool nz = false;
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-      for (int j = 0; j < 3; j++) nz |= phi[idx(p, a, x + i - 1, y + j - 1)] != R(0);
-    mask |= nz ? 1u << a : 0u;
-  }
-  used = 1u << (K - 1);
-  unsigned m = mask;
-#pragma unroll
-  for (int s = 0; s < K - 1; s++) {
-    used |= m ? 1u << s : 0u;
-    id[s] = m ? __ffs(m) - 1 : 0;
-    m &= m - 1;
-  }
-  id[K - 1] = P - 1;
-  return m == 0;
-}
-
-// Values of the K local phases; false if a value is not finite or so large
-// that products of a few of them overflow.
-template <class R>
-constexpr R kFewMax = R(sizeof(R) == 8 ? 1e50 : 1e6);
-
-template <int K, int C, class R>
-__device__ __forceinline__ bool few_load(const DevParams<R>& p, const R* __restrict__ phi, const R* __restrict__ mu,
-                                         int x, int y, const int* id, unsigned used, R (&v)[K][3][3], R* mc) {
-  bool ok = true;
-#pragma unroll
-  for (int s = 0; s < K; s++)
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-      for (int j = 0; j < 3; j++) {
-        const R w = phi[idx(p, id[s], x + i - 1, y + j - 1)];
-        v[s][i][j] = (used >> s) & 1 ? w : R(0);
-        ok &= fabs(v[s][i][j]) <= kFewMax<R>;
-      }
-#pragma unroll
-  for (int k = 0; k < C; k++) {
-    mc[k] = mu[idx(p, k, x, y)];
-    ok &= fabs(mc[k]) <= kFewMax<R>;
-  }
-  return ok;
-}
-
-// phase_cell with K local phases; false where the cell is left to phase_cell.
-template <int P, int K, int C, class R, bool NI>
-__device__ __forceinline__ bool phase_cell_few(const DevParams<R>& p, const R* __restrict__ phi,
-                                               const R* __restrict__ mu, R* __restrict__ dphi, int x, int y, R T,
-                                               const NoiseRef& nz) {
-  int id[K];
-  unsigned mask, used;
-  if (!few_phases<P, K>(p, phi, x, y, id, mask, used)) return false;
-  const SubParams<R, K> q(p, id);
-  R v[K][3][3], m[C], dp[K];
-  if (!few_load<K, C>(p, phi, mu, x, y, id, used, v, m)) return false;
-  Nbhd<K, R> n;
-  make_nbhd<K>(q, v, n);
-  const uint32_t* nzw = nz.raw ? nz.raw + nz.row_base[x] + nz.cell_off[(size_t)x * p.pitch + y] : nullptr;
-  cell_dphi<K, C, R, NI>(q, n, m, dp, T, nzw, (R)nz.amp);
-#pragma unroll
-  for (int a = 0; a < P - 1; a++)
-    if (!((mask >> a) & 1)) dphi[idx(p, a, x, y)] = R(0);
-#pragma unroll
-  for (int s = 0; s < K; s++)
-    if ((used >> s) & 1) dphi[idx(p, id[s], x, y)] = dp[s];
-  return true;
-}
-
-// load_dphi of the K local phases.
-template <int K, class R>
-__device__ __forceinline__ void few_dphi(const DevParams<R>& p, const R* __restrict__ dphi,
-                                         const signed char* __restrict__ code, int x, int y, const int* id,
-                                         unsigned used, R (&d)[K]) {
-  const bool zero = code[(size_t)x * p.pitch + y] >= 0;
-#pragma unroll
-  for (int s = 0; s < K; s++) {
-    d[s] = R(0);
-    if (!zero && ((used >> s) & 1)) d[s] = dphi[idx(p, id[s], x, y)];
-  }
-}
-
-// conc_cell_dense with K local phases; false where the cell is left to it.
-template <int P, int K, int C, class R, bool NI>
-__device__ __forceinline__ bool conc_cell_few(const DevParams<R>& p, const R* __restrict__ phi,
-                                              const R* __restrict__ mu, const R* __restrict__ dphi,
-                                              const R* __restrict__ mulo, R* __restrict__ phi_o, R* __restrict__ mu_o,
-                                              R* __restrict__ mulo_o, R tb, int tsh,
-                                              const signed char* __restrict__ code, signed char* __restrict__ oh_o,
-                                              int x, int y) {
-  const R Tc = NI ? temp_row(p, tb, y, true, tsh) : R(0);
-  const R Tr = NI ? temp_row(p, tb, y + 1, true, tsh) : R(0);
-  const R Tl = NI ? temp_row(p, tb, y - 1, true, tsh) : R(0);
-  int id[K];
-  unsigned mask, used;
-  if (!few_phases<P, K>(p, phi, x, y, id, mask, used)) return false;
-  const SubParams<R, K> q(p, id);
-  R v[K][3][3], mc[C], mf[C], mb[C], mr[C], ml[C];
-  if (!few_load<K, C>(p, phi, mu, x, y, id, used, v, mc)) return false;
-  Nbhd<K, R> nb;
-  make_nbhd<K>(q, v, nb);
-  R phc[K], phf[K], phb[K], phr[K], phl[K];
-#pragma unroll
-  for (int s = 0; s < K; s++) {
-    phc[s] = v[s][1][1];
-    phf[s] = v[s][2][1];
-    phb[s] = v[s][0][1];
-    phr[s] = v[s][1][2];
-    phl[s] = v[s][1][0];
-  }
-  R dc[K], df[K], db[K], dr[K], dl[K];
-  few_dphi<K>(p, dphi, code, x, y, id, used, dc);
-  few_dphi<K>(p, dphi, code, x + 1, y, id, used, df);
-  few_dphi<K>(p, dphi, code, x - 1, y, id, used, db);
-  few_dphi<K>(p, dphi, code, x, y + 1, id, used, dr);
-  few_dphi<K>(p, dphi, code, x, y - 1, id, used, dl);
-#pragma unroll
-  for (int k = 0; k < C; k++) {
-    mf[k] = mu[idx(p, k, x + 1, y)];
-    mb[k] = mu[idx(p, k, x - 1, y)];
-    mr[k] = mu[idx(p, k, x, y + 1)];
-    ml[k] = mu[idx(p, k, x, y - 1)];
-  }
-  R jf[C], jb[C], jr[C], jl[C];
-  face_jat<K, C, R, NI>(q, nb.gXc, nb.cYc, nb.cYf, phc, phf, mc, mf, dc, df, true, jf, Tc, Tc);
-  face_jat<K, C, R, NI>(q, nb.gXb, nb.cYb, nb.cYc, phb, phc, mb, mc, db, dc, true, jb, Tc, Tc);
-  face_jat<K, C, R, NI>(q, nb.gYc, nb.cXc, nb.cXr, phc, phr, mc, mr, dc, dr, y != p.yskip, jr, Tc, Tr);
-  face_jat<K, C, R, NI>(q, nb.gYl, nb.cXl, nb.cXc, phl, phc, ml, mc, dl, dc, (y - 1) != p.yskip, jl, Tl, Tc);
-  R Dmf[C][C], Dmb[C][C], Dmr[C][C], Dml[C][C], gmf[C], gmb[C], gmr[C], gml[C];
-  face_mob<K, C>(q, phc, phf, phb, phr, phl, mc, mf, mb, mr, ml, Dmf, Dmb, Dmr, Dml, gmf, gmb, gmr, gml);
-  R pho[K], muo[C], dmu[C];
-  cell_update<K, C, R, NI>(q, phc, mc, dc, jf, jb, jr, jl, Dmf, Dmb, Dmr, Dml, gmf, gmb, gmr, gml, pho, muo, dmu, Tc);
-#pragma unroll
-  for (int a = 0; a < P - 1; a++)
-    if (!((mask >> a) & 1)) write_with_ghosts(p, 0, phi_o + (size_t)a * p.plane, x, y, R(0));
-#pragma unroll
-  for (int s = 0; s < K; s++)
-    if ((used >> s) & 1) write_with_ghosts(p, 0, phi_o + (size_t)id[s] * p.plane, x, y, pho[s]);
-  write_mu<C, R, !Ops<R>::Exact>(p, muo, dmu, mc, mulo, mu_o, mulo_o, x, y);
-  const int o = onehot_bits<K>(pho);
-  int oh = -1;
-#pragma unroll
-  for (int s = 0; s < K; s++)
-    if (s == o) oh = id[s];
-  oh_o[(size_t)x * p.pitch + y] = (signed char)oh;
-  return true;
-}
-
 // Dense phase sweep of path 6 over the segmented phase-sweep list (written by
-// k_phase_light_oh's nbp blocks), listed cell i = first, first + stride, ...
-// Pass of a sweep in passes by the phases a cell holds (few_k): phase_cell_few
-// with that many local phases, or phase_cell in the last pass; a pass marks the
-// entries it finishes as taken (-1) and flags that it left others, without
-// which the next pass returns at once.
-template <int P, int C, class R, bool NI, int Pass>
+// k_phase_light_oh's nbp blocks): phase_cell on listed cell i, i = first,
+// first + stride, ...
+template <int P, int C, class R, bool NI>
 __device__ __forceinline__ void phase_cells_seg(const DevParams<R>& p, const R* __restrict__ phi,
-                                                const R* __restrict__ mu, R* __restrict__ dphi, int* __restrict__ lists,
-                                                int nbp, int first, int stride, R tb, int tmode, const NoiseRef& nz) {
-  constexpr int K = few_k<P, R>(Pass);
-  int* lp = lists + kSegInts;
-  if constexpr (Pass > 0) {
-    if (lists[kPhaseLeft + Pass - 1] == 0) return;
-  }
+                                                const R* __restrict__ mu, R* __restrict__ dphi,
+                                                const int* __restrict__ lists, int nbp, int first, int stride, R tb,
+                                                int tmode, const NoiseRef& nz) {
+  const int* lp = lists + kSegInts;
   const SegList<kPhaseCells> sl(lists, nbp);
-  bool left = false;
   for (int i = first; i < sl.n; i += stride) {
-    const int j = sl.seg_at(i), e = lp[j], x = e >> 16, y = e & 0xffff;
-    if (x < 2 || x > p.rx - 3 || y < 2 || y > p.ry - 3) continue;  // entries are cells of the phase sweep, or taken
-    const R T = NI ? temp_row(p, tb, y, (tmode & 1) != 0, tmode >> 1) : R(0);
-    if constexpr (K > 0) {
-      const bool done = phase_cell_few<P, K, C, R, NI>(p, phi, mu, dphi, x, y, T, nz);
-      if (done) lp[j] = -1;
-      left = left || !done;
-    } else {
-      phase_cell<P, C, R, NI>(p, phi, mu, dphi, x, y, T, nz);
-    }
+    const int e = lp[sl.seg_at(i)], x = e >> 16, y = e & 0xffff;
+    if (x < 2 || x > p.rx - 3 || y < 2 || y > p.ry - 3) continue;  // entries are cells of the phase sweep
+    phase_cell<P, C, R, NI>(p, phi, mu, dphi, x, y, NI ? temp_row(p, tb, y, (tmode & 1) != 0, tmode >> 1) : R(0), nz);
   }
-  if (left) lists[kPhaseLeft + Pass] = 1;
 }
 
 // Dense phase sweep and light mu sweep of path 6 in one launch of BX x BY
@@ -1290,9 +1097,8 @@ __global__ void __launch_bounds__(BX * BY) __attribute__((amdgpu_waves_per_eu(GP
                     int tmode, int tsh, NoiseRef nz) {
   const DevParams<R>& p = *prm;
   if ((int)blockIdx.x < nd) {
-    phase_cells_seg<P, C, R, NI, 0>(p, phi, mu, dphi, lists, nbp,
-                                        blockIdx.x * (BX * BY) + threadIdx.y * BX + threadIdx.x, nd * (BX * BY), tb,
-                                        tmode, nz);
+    phase_cells_seg<P, C, R, NI>(p, phi, mu, dphi, lists, nbp, blockIdx.x * (BX * BY) + threadIdx.y * BX + threadIdx.x,
+                                 nd * (BX * BY), tb, tmode, nz);
     return;
   }
   const int L = blockIdx.x - nd, n = gridDim.x - nd;
@@ -1306,12 +1112,13 @@ __global__ void __launch_bounds__(BX * BY) __attribute__((amdgpu_waves_per_eu(GP
 // own register budget): the dense phase sweep on a 1-D grid of 256-lane
 // blocks, then the light mu sweep on the gx x gy grid.  The one-hot path uses
 // them where onehot_wide holds.
-template <int P, int C, class R, bool NI, int Pass>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(onehot_dense_waves<P, R>(Pass))))
-    k_phase_cells_oh(const DevParams<R>* __restrict__ prm, const R* __restrict__ phi, const R* __restrict__ mu,
-                     R* __restrict__ dphi, int* __restrict__ lists, int nbp, R tb, int tmode, NoiseRef nz) {
-  phase_cells_seg<P, C, R, NI, Pass>(*prm, phi, mu, dphi, lists, nbp, blockIdx.x * 256 + threadIdx.x, gridDim.x * 256,
-                                     tb, tmode, nz);
+template <int P, int C, class R, bool NI = false>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(onehot_dense_waves<P, R>()))) k_phase_cells_oh(const DevParams<R>* __restrict__ prm,
+                                                                 const R* __restrict__ phi, const R* __restrict__ mu,
+                                                                 R* __restrict__ dphi, const int* __restrict__ lists,
+                                                                 int nbp, R tb, int tmode, NoiseRef nz) {
+  phase_cells_seg<P, C, R, NI>(*prm, phi, mu, dphi, lists, nbp, blockIdx.x * 256 + threadIdx.x, gridDim.x * 256, tb,
+                               tmode, nz);
 }
 
 template <int P, int C, class R, bool NI = false>
@@ -1328,32 +1135,6 @@ __global__ void __launch_bounds__(BX * BY) k_conc_light_oh(const DevParams<R>* _
                               mulo_o, oh_o, lists + kSegInts + capp, lists + kSegs * kSegStride, tb, tsh);
 }
 
-// Pass of the dense mu sweep of path 6 over the cells of few phases, one lane
-// per listed cell: conc_cell_few, marking and flagging as phase_cells_seg does.
-template <int P, int C, class R, bool NI, int Pass>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(onehot_dense_waves<P, R>(Pass))))
-    k_conc_cells_few(const DevParams<R>* __restrict__ prm, const R* __restrict__ phi, const R* __restrict__ mu,
-                     const R* __restrict__ dphi, const R* __restrict__ mulo, R* __restrict__ phi_o,
-                     R* __restrict__ mu_o, R* __restrict__ mulo_o, R tb, int tsh, int* __restrict__ lists, int capp,
-                     int nbc, const signed char* __restrict__ code, signed char* __restrict__ oh_o) {
-  if constexpr (Pass > 0) {
-    if (lists[kMuLeft + Pass - 1] == 0) return;
-  }
-  const DevParams<R>& p = *prm;
-  int* lc = lists + kSegInts + capp;
-  const SegList<kMuCells> sl(lists + kSegs * kSegStride, nbc);
-  bool left = false;
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < sl.n; i += gridDim.x * 256) {
-    const int j = sl.seg_at(i), e = lc[j], x = e >> 16, y = e & 0xffff;
-    if (x < 3 || x > p.mesh_x + 2 || y < 3 || y > p.mesh_y + 2) continue;  // entries are interior cells
-    const bool done = conc_cell_few<P, few_k<P, R>(Pass), C, R, NI>(p, phi, mu, dphi, mulo, phi_o, mu_o, mulo_o, tb, tsh,
-                                                                code, oh_o, x, y);
-    if (done) lc[j] = -1;
-    left = left || !done;
-  }
-  if (left) lists[kMuLeft + Pass] = 1;
-}
-
 // Dense mu sweep of path 6: the update of conc_cell_dense, with the new
 // one-hot codes into oh_o, on the cells of the segmented mu-sweep list
 // (written by the nbc light blocks of the mu sweep); one lane per cell where
@@ -1366,7 +1147,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(onehot
 // conc_cell_dense, so the bits are unchanged.  Clears the phase-sweep
 // counters, whose readers have finished.
 template <int P, int C, class R, bool NI = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(onehot_dense_waves<P, R>(few_passes<P, R>())))) k_conc_cells_oh(const DevParams<R>* __restrict__ prm,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(onehot_dense_waves<P, R>()))) k_conc_cells_oh(const DevParams<R>* __restrict__ prm,
                                                                 const R* __restrict__ phi, const R* __restrict__ mu,
                                                                 const R* __restrict__ dphi,
                                                                 const R* __restrict__ mulo, R* __restrict__ phi_o,
@@ -1379,10 +1160,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(onehot
   const int* lc = lists + kSegInts + capp;
   const SegList<kMuCells> sl(lists + kSegs * kSegStride, nbc);
   if (blockIdx.x == 0 && threadIdx.x < kSegs) lists[kSegStride * threadIdx.x] = 0;
-  if (blockIdx.x == 0 && threadIdx.x < kFewPasses) lists[kPhaseLeft + threadIdx.x] = 0;
-  if constexpr (few_passes<P, R>() > 0) {
-    if (lists[kMuLeft + few_passes<P, R>() - 1] == 0) return;  // the passes before took every cell
-  }
   if constexpr (onehot_conc_one_lane<P, R>()) {  // one lane per listed cell
     for (int i = blockIdx.x * 256 + threadIdx.x; i < sl.n; i += gridDim.x * 256) {
       const int e = lc[sl.seg_at(i)], x = e >> 16, y = e & 0xffff;

@@ -35,21 +35,6 @@
 
 namespace GPK_NS {
 
-// Local phases of pass i of the one-hot path's dense sweeps by the phases a
-// cell holds (few_phases); 0: the pass takes the full P.  Four (three solids
-// and the liquid) hold nearly every cell; from eight phases on a pass of six
-// takes the cells around a fourth grain, since a single such cell in the full
-// kernels costs their whole latency (4096^2, nine phases: 94 and 92 us for what
-// the pass of six does in 63 and 79; a pass with nothing left takes 5).  Binary64
-// only: in binary32 solved phases keep values of the order of the rounding, so
-// that many cells hold all phases, and the sums would be contracted
-// differently.
-constexpr int kFewPasses = 2;  // at most
-template <int P, class R>
-constexpr int few_passes() { return sizeof(R) != 8 || P < 5 ? 0 : P < 8 ? 1 : 2; }
-template <int P, class R>
-constexpr int few_k(int pass) { return pass >= few_passes<P, R>() ? 0 : pass == 0 ? 4 : 6; }
-
 // At nine or more phases the one-hot path runs its dense phase sweep as a
 // launch of its own, so that the light mu sweep is not held to the dense
 // sweep's register budget (4096^2, 9 phases, binary32: 1.49e10 -> 1.64e10
@@ -61,11 +46,9 @@ constexpr int few_k(int pass) { return pass >= few_passes<P, R>() ? 0 : pass == 
 // the light waves at six phases were held to the dense pass's two per SIMD (64
 // us at 1531 x 1021, against 42 + 21 us for the two launches).
 template <int P, class R>
-constexpr bool onehot_wide() { return P >= 9 || few_passes<P, R>() > 0; }
+constexpr bool onehot_wide() { return P >= 9; }
 template <int P, class R>
-constexpr int onehot_dense_waves(int pass) {
-  return sizeof(R) == 8 && (few_k<P, R>(pass) == 6 || (P >= 9 && few_k<P, R>(pass) == 0)) ? 1 : GP_WAVES_PER_EU;
-}
+constexpr int onehot_dense_waves() { return onehot_wide<P, R>() && sizeof(R) == 8 ? 1 : GP_WAVES_PER_EU; }
 // The one-hot path's dense mu sweep takes two waves per listed cell (the x and
 // y antitrapping faces side by side) below nine phases, one lane per cell from
 // nine: at 4096^2 and nine phases one lane is 15% (binary64) and 6% (binary32)
@@ -188,56 +171,6 @@ __device__ __forceinline__ void phase_cell(const DevParams<R>& p, const R* __res
   for (int a = 0; a < P; a++) dphi[idx(p, a, x, y)] = dp[a];
 }
 
-// Face mobilities and mu gradients of a cell (calculate_gradients.h:148-165).
-template <int P, int C, class R, class Pm>
-__device__ __forceinline__ void face_mob(const Pm& p, const R* phc, const R* phf, const R* phb, const R* phr,
-                                         const R* phl, const R* mc, const R* mf, const R* mb, const R* mr, const R* ml,
-                                         R (&Dmf)[C][C], R (&Dmb)[C][C], R (&Dmr)[C][C], R (&Dml)[C][C], R* gmf,
-                                         R* gmb, R* gmr, R* gml) {
-  R Dc[C][C], Df[C][C], Db[C][C], Dr[C][C], Dl[C][C];
-  cell_D<P, C>(p, phc, Dc);
-  cell_D<P, C>(p, phf, Df);
-  cell_D<P, C>(p, phb, Db);
-  cell_D<P, C>(p, phr, Dr);
-  cell_D<P, C>(p, phl, Dl);
-#pragma unroll
-  for (int k = 0; k < C; k++) {
-#pragma unroll
-    for (int l = 0; l < C; l++) {
-      Dmf[k][l] = (Df[k][l] + Dc[k][l]) * R(0.5);
-      Dmb[k][l] = (Dc[k][l] + Db[k][l]) * R(0.5);
-      Dmr[k][l] = (Dr[k][l] + Dc[k][l]) * R(0.5);
-      Dml[k][l] = (Dc[k][l] + Dl[k][l]) * R(0.5);
-    }
-    gmf[k] = div_dx(mf[k] - mc[k], p);
-    gmb[k] = div_dx(mc[k] - mb[k], p);
-    gmr[k] = div_dy(mr[k] - mc[k], p);
-    gml[k] = div_dy(mc[k] - ml[k], p);
-  }
-}
-
-// Writes the new mu of a cell with its ghost images; Kahan adds the mu
-// increment to mu + mulo (binary32).
-template <int C, class R, bool Kahan>
-__device__ __forceinline__ void write_mu(const DevParams<R>& p, const R* muo, const R* dmu, const R* mc,
-                                         const R* __restrict__ mulo, R* __restrict__ mu_o, R* __restrict__ mulo_o,
-                                         int x, int y) {
-  if constexpr (!Kahan) {
-#pragma unroll
-    for (int k = 0; k < C; k++) write_with_ghosts(p, 1, mu_o + (size_t)k * p.plane, x, y, muo[k]);
-  } else {
-#pragma unroll
-    for (int k = 0; k < C; k++) {
-      R lo = mulo[idx(p, k, x, y)];
-      R yk = dmu[k] - lo;
-      R t = mc[k] + yk;
-      R lo_n = (t - mc[k]) - yk;
-      write_with_ghosts(p, 1, mu_o + (size_t)k * p.plane, x, y, t);
-      mulo_o[idx(p, k, x, y)] = lo_n;
-    }
-  }
-}
-
 // mu and phi update of interior cell (x,y) from its 3x3 phi block v, the mu of
 // its five-point stencil, its delta-phi and the antitrapping fluxes of its four
 // faces; writes the cell and its ghost images.  Kahan adds the mu increment to
@@ -258,8 +191,28 @@ __device__ __forceinline__ int conc_apply(const DevParams<R>& p, const R (&v)[P]
     phr[a] = v[a][1][2];
     phl[a] = v[a][1][0];
   }
+  // face mobilities and mu gradients (calculate_gradients.h:148-165)
+  R Dc[C][C], Df[C][C], Db[C][C], Dr[C][C], Dl[C][C];
+  cell_D<P, C>(p, phc, Dc);
+  cell_D<P, C>(p, phf, Df);
+  cell_D<P, C>(p, phb, Db);
+  cell_D<P, C>(p, phr, Dr);
+  cell_D<P, C>(p, phl, Dl);
   R Dmf[C][C], Dmb[C][C], Dmr[C][C], Dml[C][C], gmf[C], gmb[C], gmr[C], gml[C];
-  face_mob<P, C>(p, phc, phf, phb, phr, phl, mc, mf, mb, mr, ml, Dmf, Dmb, Dmr, Dml, gmf, gmb, gmr, gml);
+#pragma unroll
+  for (int k = 0; k < C; k++) {
+#pragma unroll
+    for (int l = 0; l < C; l++) {
+      Dmf[k][l] = (Df[k][l] + Dc[k][l]) * R(0.5);
+      Dmb[k][l] = (Dc[k][l] + Db[k][l]) * R(0.5);
+      Dmr[k][l] = (Dr[k][l] + Dc[k][l]) * R(0.5);
+      Dml[k][l] = (Dc[k][l] + Dl[k][l]) * R(0.5);
+    }
+    gmf[k] = div_dx(mf[k] - mc[k], p);
+    gmb[k] = div_dx(mc[k] - mb[k], p);
+    gmr[k] = div_dy(mr[k] - mc[k], p);
+    gml[k] = div_dy(mc[k] - ml[k], p);
+  }
   R pho[P], muo[C], dmu[C];
   if (comp) {  // composition field, updated in place (each cell reads only its own)
     R cst[C];
@@ -274,7 +227,20 @@ __device__ __forceinline__ int conc_apply(const DevParams<R>& p, const R (&v)[P]
   }
 #pragma unroll
   for (int a = 0; a < P; a++) write_with_ghosts(p, 0, phi_o + (size_t)a * p.plane, x, y, pho[a]);
-  write_mu<C, R, Kahan>(p, muo, dmu, mc, mulo, mu_o, mulo_o, x, y);
+  if constexpr (!Kahan) {
+#pragma unroll
+    for (int k = 0; k < C; k++) write_with_ghosts(p, 1, mu_o + (size_t)k * p.plane, x, y, muo[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < C; k++) {
+      R lo = mulo[idx(p, k, x, y)];
+      R yk = dmu[k] - lo;
+      R t = mc[k] + yk;
+      R lo_n = (t - mc[k]) - yk;
+      write_with_ghosts(p, 1, mu_o + (size_t)k * p.plane, x, y, t);
+      mulo_o[idx(p, k, x, y)] = lo_n;
+    }
+  }
   int a1 = -1, n1 = 0, nz = 0;  // the exact one-hot bits
 #pragma unroll
   for (int a = 0; a < P; a++) {

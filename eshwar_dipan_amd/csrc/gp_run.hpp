@@ -377,29 +377,6 @@ int run_compact(gp_ctx *c, long nsteps) {
   return run_compact_in<P, C, R, NI>(c, nsteps, c->dcells);
 }
 
-// The passes of the one-hot path's dense phase sweep, and those of its dense mu
-// sweep over cells of few phases (few_k); k_conc_cells_oh follows the latter.
-template <int P, int C, class R, bool NI, int Pass = 0>
-void phase_passes(gp_ctx *c, int grid, const DevParams<R> *prm, const R *phi, const R *mu, R *dphi, int nbp, R tb,
-                  int tmode, const NoiseRef &nz) {
-  hipLaunchKernelGGL((k_phase_cells_oh<P, C, R, NI, Pass>), dim3(grid), dim3(256), 0, c->stream, prm, phi, mu, dphi,
-                     c->dcells6, nbp, tb, tmode, nz);
-  if constexpr (Pass < few_passes<P, R>())
-    phase_passes<P, C, R, NI, Pass + 1>(c, grid, prm, phi, mu, dphi, nbp, tb, tmode, nz);
-}
-
-template <int P, int C, class R, bool NI, int Pass = 0>
-void conc_few_passes(gp_ctx *c, int grid, const DevParams<R> *prm, const R *phi, const R *mu, const R *dphi,
-                     const R *mulo, R *phi_o, R *mu_o, R *mulo_o, R tb, int tsh, int capp, int nbc,
-                     signed char *oh_o) {
-  if constexpr (Pass < few_passes<P, R>()) {
-    hipLaunchKernelGGL((k_conc_cells_few<P, C, R, NI, Pass>), dim3(grid), dim3(256), 0, c->stream, prm, phi, mu, dphi,
-                       mulo, phi_o, mu_o, mulo_o, tb, tsh, c->dcells6, capp, nbc, (const signed char *)c->dcode, oh_o);
-    conc_few_passes<P, C, R, NI, Pass + 1>(c, grid, prm, phi, mu, dphi, mulo, phi_o, mu_o, mulo_o, tb, tsh, capp, nbc,
-                                           oh_o);
-  }
-}
-
 // Steps of the one-hot path (6): per step k_phase_light_oh, k_phase_conc_oh
 // (the dense phase sweep on its first nd blocks, the light mu sweep on the
 // rest) and k_conc_cells_oh with the one-hot plane of the output buffer.  The
@@ -454,13 +431,12 @@ int run_onehot(gp_ctx *c, long nsteps) {
                          (const signed char *)c->dcode, phi_o, mu_o, mulo_o, oh[c->cur ^ 1], c->dcells6, nbp, capp,
                          nd, gx, tb, tmode, tsh, nz);
     } else {
-      phase_passes<P, C, R, NI>(c, nd, prm, phi, mu, dphi, nbp, tb, tmode, nz);
+      hipLaunchKernelGGL((k_phase_cells_oh<P, C, R, NI>), dim3(nd), dim3(256), 0, c->stream, prm, phi, mu, dphi,
+                         (const int *)c->dcells6, nbp, tb, tmode, nz);
       hipLaunchKernelGGL((k_conc_light_oh<P, C, R, NI>), dim3(gx, gy), blk, 0, c->stream, prm, mu, mulo,
                          (const signed char *)c->dcode, phi_o, mu_o, mulo_o, oh[c->cur ^ 1], c->dcells6, capp, tb,
                          tsh);
     }
-    conc_few_passes<P, C, R, NI>(c, gdense, prm, phi, mu, dphi, mulo, phi_o, mu_o, mulo_o, tb, tsh, capp, nbc,
-                                 oh[c->cur ^ 1]);
     hipLaunchKernelGGL((k_conc_cells_oh<P, C, R, NI>), dim3(gdense), dim3(256), 0, c->stream, prm, phi, mu,
                        (const R *)dphi, mulo, phi_o, mu_o, mulo_o, tb, tsh, c->dcells6, capp, nbc,
                        (const signed char *)c->dcode, oh[c->cur ^ 1]);
