@@ -333,8 +333,10 @@ __device__ __forceinline__ void bulk_cell(const DevParams<R>& p, const R* __rest
 // Bulk tiles: the tile and its 2-cell halo hold the exact one-hot vector of
 // phase flag_i (onehot_bits), so every cell satisfies the bulk_cell conditions.
 // The phase vector is known from the flag: phi is not read, and its planes are
-// written only where the output buffer does not hold the same vector already
-// (flag_o describes the state of two steps back until it is overwritten here).
+// written only where the output buffer does not hold the same vector already, at
+// the cells and at their ghost images (flag_o describes the state of two steps
+// back until it is overwritten here; the sweeps that set it write both, k_flags
+// looks at both).
 // The sweep is bound by memory and now moves the mu planes alone: on 64 grids of
 // 64^2 to 512^2 (two phases, binary64) 143 -> 58 us a step, 100 MB at 1.7 TB/s.
 template <int P, int C, class R, int TX, int TY>
@@ -1416,8 +1418,36 @@ __global__ void k_clear_counts(int* __restrict__ cnt) {
   if (threadIdx.x < 4) cnt[threadIdx.x] = 0;
 }
 
-// Flags of a freshly loaded state (one block per tile); those of the other
-// buffer, of unknown contents, are cleared.
+// Whether every phi ghost image of interior cell (x, y) holds the exact one-hot
+// vector of phase f.  After a frame shift the ghost layers are not images: the
+// rows were moved as they lay, and no boundary copy followed.
+template <int P, class R>
+__device__ __forceinline__ bool ghosts_hold(const DevParams<R>& p, const R* __restrict__ phi, int x, int y, int f) {
+  if (x >= p.gfree[0][0][0] && x <= p.gfree[0][0][1] && y >= p.gfree[0][1][0] && y <= p.gfree[0][1][1]) return true;
+  bool held = true;
+#pragma unroll 1
+  for (int i = -1; i < 6; i++) {  // x itself, then its images
+    if (i >= 0 && p.gsrc[0][0][i] != x) continue;
+    const int gx = i < 0 ? x : ghost_index(i, p.rx);
+#pragma unroll 1
+    for (int j = -1; j < 6; j++) {
+      if (j >= 0 && p.gsrc[0][1][j] != y) continue;
+      const int gy = j < 0 ? y : ghost_index(j, p.ry);
+      R ph[P];
+#pragma unroll
+      for (int a = 0; a < P; a++) ph[a] = phi[idx(p, a, gx, gy)];
+      held = held && onehot_bits<P>(ph) == f;
+    }
+  }
+  return held;
+}
+
+// Flags of a state that no step of the tile paths left (one block per tile);
+// those of the other buffer, of unknown contents, are cleared.  A flag vouches
+// for the tile's cells and for their ghost images: k_plan takes a ghost cell for
+// its source, and k_bulk leaves both unwritten where the flag is the phase it
+// would write.  A tile whose images differ is an interface tile for one step,
+// which reads the ghost layers as they are.
 template <int P, class R, int TX, int TY>
 __global__ void __launch_bounds__(256) k_flags(const Inst<R>* __restrict__ inst, const int* __restrict__ tinst,
                                                int par, int* __restrict__ flag, int* __restrict__ flag_x) {
@@ -1435,7 +1465,8 @@ __global__ void __launch_bounds__(256) k_flags(const Inst<R>* __restrict__ inst,
     R ph[P];
 #pragma unroll
     for (int a = 0; a < P; a++) ph[a] = phi[idx(p, a, x, y)];
-    f = flag_combine(f, onehot_bits<P>(ph));
+    const int cf = onehot_bits<P>(ph);
+    f = flag_combine(f, cf >= 0 && !ghosts_hold<P>(p, phi, x, y, cf) ? -1 : cf);
   }
   f = block_flag(f, red);
   if (threadIdx.x == 0) {
