@@ -827,9 +827,10 @@ struct SegList {
 
 // oh of the current buffer from its interior cells, oh of the other buffer
 // unknown (-1): the set-up after a step of another path or a new state.  A
-// cell with ghost images (within 3 cells of a face) is left unknown, so that
-// only a write of the cell and its images by this path's own sweeps vouches
-// for them.
+// cell that may have ghost images (outside the band that is the source of none:
+// the copies of Neumann and periodic faces reach the fourth row from the face)
+// is left unknown, so that only a write of the cell and its images by this
+// path's own sweeps vouches for them.
 template <int P, class R>
 __global__ void __launch_bounds__(BX * BY) k_oh_prime(const DevParams<R>* __restrict__ prm, const R* __restrict__ phi,
                                                       signed char* __restrict__ oh, signed char* __restrict__ oh_x) {
@@ -843,7 +844,7 @@ __global__ void __launch_bounds__(BX * BY) k_oh_prime(const DevParams<R>* __rest
 #pragma unroll
   for (int a = 0; a < P; a++) ph[a] = phi[idx(p, a, x, y)];
   const size_t i = (size_t)x * p.pitch + y;
-  const bool edge = x < 6 || x > p.mesh_x - 1 || y < 6 || y > p.mesh_y - 1;
+  const bool edge = x < p.gfree[0][0][0] || x > p.gfree[0][0][1] || y < p.gfree[0][1][0] || y > p.gfree[0][1][1];
   oh[i] = (signed char)(edge ? -1 : onehot_bits<P>(ph));
   oh_x[i] = -1;
 }

@@ -90,3 +90,18 @@ def _outermost(path, dtype):
         assert pos == opos, (n, pos, opos)
         if dtype == "f64":
             assert max(float(np.abs(g[k] - o[k]).max()) for k in (0, 1)) <= TOL64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_gpu_onehot_outermost_ghosts_after_shift(dtype):
+    print(f"\n[gpu] shift leaves another phase in the outermost ghost row, path 6, {dtype}", flush=True)
+    _outermost(6, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first", [1, 2, 33])
+def test_gpu_onehot_after_shift_over_another_phase(first):
+    print(f"\n[gpu] shift leaves another phase in the low ghosts, path 6, {first} steps first", flush=True)
+    inp = gputil.make_params(P=3, C=1, mesh=(41, 210), aniso=0.02, gabc=1.0, bc=(1, 1, 1, 1))
+    _check(inp, _layout(inp, below=1, phase=0, rows=D), 6, [(6, first), (1, 1), (6, 2), (6, 32), (1, 2)])
