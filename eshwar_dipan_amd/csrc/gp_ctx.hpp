@@ -84,7 +84,12 @@ struct gp_ctx {
   long path_steps[GP_NPATHS];  // steps run per kernel path since the last gp_path_steps reset
   int shape;             // tile shape of the sparse two-pass path (index into the candidate list)
   int shape_set;         // tile shape the tile set was built for (-1: none)
-  double *stage;        // gp_set_state / gp_get_state: fields in transit (on first use), held under stage_mu
+  // gp_set_state / gp_get_state: the context whose buffer for fields in transit
+  // this one uses (itself; the master for an ensemble member), that buffer (on
+  // first use), its size (0: none is kept) and the lock under which a call uses it
+  gp_ctx *stage_of;
+  double *stage;
+  size_t stage_bytes;
   std::mutex stage_mu;
 };
 

@@ -194,7 +194,11 @@ void gp_destroy(gp_ctx *ctx);
 
 /* Load / read back the interior fields (host arrays in the layout above, binary64).
    gp_set_state also fills the ghost layers, like apply_boundary_conditions(0)
-   after fill_domain / restart reading (microsim_gp.c:48-57,84). */
+   after fill_domain / restart reading (microsim_gp.c:48-57,84).  The fields
+   pass through P + C binary64 planes of device memory: a context that needs at
+   most GP_TRANSIT_KEEP bytes for them keeps them from its first call until it is
+   destroyed; a larger one gives them back before the call returns. */
+#define GP_TRANSIT_KEEP (8u << 20)
 int  gp_set_state(gp_ctx *ctx, const double *phi, const double *mu);
 int  gp_get_state(gp_ctx *ctx, double *phi, double *mu);
 
@@ -304,6 +308,10 @@ int  gp_autotune(gp_ctx *ctx, long steps, int *path, int *shape);
  * 32 steps are replayed as one captured HIP graph.  Member i is addressed by
  * its index; its state and statistics work as for a context.  Each member's
  * binary64 results equal those of a context of its own.
+ *
+ * The members share one buffer for fields in transit (gp_set_state above), as
+ * large as the largest member among those within GP_TRANSIT_KEEP needs; calls on
+ * different members from several threads take turns on it.
  */
 typedef struct gp_ensemble gp_ensemble;
 int  gp_ensemble_create(const gp_params *params, int n, int dtype, gp_ensemble **out);
