@@ -83,52 +83,28 @@ struct DevParams {
   unsigned long long lcg_step[2];        // the map of one step's (rows_x-2)(rows_y-2) draws
 };
 
-// The parameters of K of the phases under local indices 0..K-1: the cell
-// functions below take DevParams or this view of it, in which table [a][b] is
-// the full table at [id[a]][id[b]].  The indices are per lane, so the entries
-// come through vector loads (a few KB, resident in L1) where DevParams' come
-// through scalar ones.  id is an array beside the view, not in it: a view that
-// held its own address would stay in scratch.
+// The parameters of one phase, a, for cell_update of a cell that holds that phase
+// alone: cell_update<1> and the functions it calls take DevParams or this view of
+// it, in which every phase index stands for a.  The phase may differ from lane to
+// lane, so the entries come through vector loads (a few KB, resident in L1) where
+// DevParams' come through scalar ones.
 template <class T>
-struct SubRow {
+struct PhaseRow {
   const T* t;
-  const int* id;
-  __device__ __forceinline__ const T& operator[](int a) const { return t[id[a]]; }
-};
-template <class T>
-struct SubTab {
-  const T (*t)[PM];
-  const int* id;
-  __device__ __forceinline__ SubRow<T> operator[](int a) const { return SubRow<T>{t[id[a]], id}; }
-};
-template <class T>
-struct SubCube {
-  const T (*t)[PM][PM];
-  const int* id;
-  __device__ __forceinline__ SubTab<T> operator[](int a) const { return SubTab<T>{t[id[a]], id}; }
+  int a;
+  __device__ __forceinline__ const T& operator[](int) const { return t[a]; }
 };
 
-template <class R, int K>
-struct SubParams {
-  const int &obstacle, &anisotropy, &mu_solver, &pair_sym, &pow2_dx, &pow2_dy, &mpi, &mpi_noise;
-  const R &dx, &dy, &dt, &two_dy, &inv_dx, &inv_dy, &inv_two_dy, &epsilon, &inv_eps, &tau, &w_pref, &jscale, &well_at,
-      &Teq, &tgv, &V;
-  SubTab<R> gamma, tau_ab, dab;
-  SubCube<R> gamma_abc;
-  SubTab<R[2][2]> rot, rot_inv;
-  SubRow<R[CM]> at_coef, Bsh, B, Beq, dBbdT, dC, ceqL, ceqS;
-  SubRow<R[CM][CM]> A, cmu;
-  SubRow<R[CM][CM][CM]> dcm;
-  SubRow<R> Cf, dTs, dTl;
-  __device__ __forceinline__ SubParams(const DevParams<R>& f, const int (&id)[K])
-      : obstacle(f.obstacle), anisotropy(f.anisotropy), mu_solver(f.mu_solver), pair_sym(f.pair_sym),
-        pow2_dx(f.pow2_dx), pow2_dy(f.pow2_dy), mpi(f.mpi), mpi_noise(f.mpi_noise), dx(f.dx), dy(f.dy), dt(f.dt),
-        two_dy(f.two_dy), inv_dx(f.inv_dx), inv_dy(f.inv_dy), inv_two_dy(f.inv_two_dy), epsilon(f.epsilon),
-        inv_eps(f.inv_eps), tau(f.tau), w_pref(f.w_pref), jscale(f.jscale), well_at(f.well_at), Teq(f.Teq),
-        tgv(f.tgv), V(f.V), gamma{f.gamma, id}, tau_ab{f.tau_ab, id}, dab{f.dab, id}, gamma_abc{f.gamma_abc, id},
-        rot{f.rot, id}, rot_inv{f.rot_inv, id}, at_coef{f.at_coef, id}, Bsh{f.Bsh, id}, B{f.B, id}, Beq{f.Beq, id},
-        dBbdT{f.dBbdT, id}, dC{f.dC, id}, ceqL{f.ceqL, id}, ceqS{f.ceqS, id}, A{f.A, id}, cmu{f.cmu, id},
-        dcm{f.dcm, id}, Cf{f.Cf, id}, dTs{f.dTs, id}, dTl{f.dTl, id} {}
+template <class R>
+struct PhaseParams {
+  const int &mu_solver, &pow2_dx, &pow2_dy;
+  const R &dx, &dy, &dt, &inv_dx, &inv_dy, &jscale, &Teq, &tgv;
+  PhaseRow<R[CM]> Bsh, Beq, dBbdT;
+  PhaseRow<R[CM][CM]> A, cmu;
+  __device__ __forceinline__ PhaseParams(const DevParams<R>& f, int a)
+      : mu_solver(f.mu_solver), pow2_dx(f.pow2_dx), pow2_dy(f.pow2_dy), dx(f.dx), dy(f.dy), dt(f.dt),
+        inv_dx(f.inv_dx), inv_dy(f.inv_dy), jscale(f.jscale), Teq(f.Teq), tgv(f.tgv), Bsh{f.Bsh, a}, Beq{f.Beq, a},
+        dBbdT{f.dBbdT, a}, A{f.A, a}, cmu{f.cmu, a} {}
 };
 
 // drand48's generator: x' = (0x5DEECE66D x + 0xB) mod 2^48, value x' 2^-48
@@ -178,8 +154,8 @@ __device__ __forceinline__ R div_dy(R v, const Pm& p) {
   if constexpr (Ops<R>::Exact) return p.pow2_dy ? v * p.inv_dy : v / p.dy; else return v * p.inv_dy;
 #endif
 }
-template <class R, class Pm>
-__device__ __forceinline__ R div_2dy(R v, const Pm& p) {
+template <class R>
+__device__ __forceinline__ R div_2dy(R v, const DevParams<R>& p) {
   #ifdef GP_POW2
   return v * p.inv_two_dy;
 #else
@@ -215,8 +191,8 @@ __device__ __forceinline__ R Mu_of_c(const Pm& p, const R* c, int a, int i) {
 }
 
 // f_a(c)  (functionF_01.h:5-18)
-template <int C, class R, class Pm>
-__device__ __forceinline__ R free_energy(const Pm& p, const R* c, int a) {
+template <int C, class R>
+__device__ __forceinline__ R free_energy(const DevParams<R>& p, const R* c, int a) {
   R s = R(0);
 #pragma unroll
   for (int i = 0; i < C; i++) {
@@ -264,8 +240,8 @@ __device__ __forceinline__ R dhphi(const R* ph, int b, int a) {
 }
 
 // psi_b(mu) = f_b(c_b(mu)) - mu.c_b(mu)  (functionF_01.h:41-57, the b-term of dpsi)
-template <int C, class R, class Pm>
-__device__ __forceinline__ R psi_of_mu(const Pm& p, const R* mu, int b) {
+template <int C, class R>
+__device__ __forceinline__ R psi_of_mu(const DevParams<R>& p, const R* mu, int b) {
   R c[C];
   R psi = R(0);
 #pragma unroll
@@ -278,8 +254,8 @@ __device__ __forceinline__ R psi_of_mu(const Pm& p, const R* mu, int b) {
 }
 
 // tau(phi)  (functionTau.h:1-16)
-template <int P, class R, class Pm>
-__device__ __forceinline__ R tau_phi(const Pm& p, const R* ph) {
+template <int P, class R>
+__device__ __forceinline__ R tau_phi(const DevParams<R>& p, const R* ph) {
   R s = R(0), s1 = R(0);
 #pragma unroll
   for (int a = 0; a < P; a++)
@@ -339,8 +315,8 @@ __device__ __forceinline__ R Mu_of_c_t(const Pm& p, const R* c, int a, int i, R 
 
 // B_a,i(T) and C_a(T) (functionF_01.h:62-104), the tables init_propertymatrices(T)
 // leaves for the phase-field terms of a cell of temperature T
-template <int C, class R, class Pm>
-__device__ __forceinline__ R B_of_T(const Pm& p, int L, R T, int i, int a) {
+template <int C, class R>
+__device__ __forceinline__ R B_of_T(const DevParams<R>& p, int L, R T, int i, int a) {
   if (a == L) return R(0);
   R cl[C], cs[C], sum_c = R(0);
 #pragma unroll
@@ -352,8 +328,8 @@ __device__ __forceinline__ R B_of_T(const Pm& p, int L, R T, int i, int a) {
   return (R(2.0) * (p.A[L][i][i] * cl[i] - p.A[a][i][i] * cs[i]) + sum_c);
 }
 
-template <int C, class R, class Pm>
-__device__ __forceinline__ R C_of_T(const Pm& p, int L, R T, int a) {
+template <int C, class R>
+__device__ __forceinline__ R C_of_T(const DevParams<R>& p, int L, R T, int a) {
   if (a == L) return R(0);
   R cl[C], cs[C], sum_c = R(0);
 #pragma unroll
@@ -369,8 +345,8 @@ __device__ __forceinline__ R C_of_T(const Pm& p, int L, R T, int a) {
   return sum_c;
 }
 
-template <int P, int C, class R, class Pm>
-__device__ __forceinline__ R psi_of_mu_t(const Pm& p, const R* mu, int b, R T) {
+template <int P, int C, class R>
+__device__ __forceinline__ R psi_of_mu_t(const DevParams<R>& p, const R* mu, int b, R T) {
   R c[C];
   R psi = R(0);
 #pragma unroll
@@ -403,8 +379,8 @@ __device__ __forceinline__ R Mu_of_c_(const Pm& p, const R* c, int a, int i, R T
   if constexpr (NI) return Mu_of_c_t<C>(p, c, a, i, T);
   else return Mu_of_c<C>(p, c, a, i);
 }
-template <int P, int C, bool NI, class R, class Pm>
-__device__ __forceinline__ R psi_of_mu_(const Pm& p, const R* mu, int b, R T) {
+template <int P, int C, bool NI, class R>
+__device__ __forceinline__ R psi_of_mu_(const DevParams<R>& p, const R* mu, int b, R T) {
   if constexpr (NI) return psi_of_mu_t<P, C>(p, mu, b, T);
   else return psi_of_mu<C>(p, mu, b);
 }
@@ -475,8 +451,8 @@ struct Nbhd {
   bool present[P];         // phase b is nonzero somewhere in the 3x3 block
 };
 
-template <int P, class R, class Pm>
-__device__ __forceinline__ void make_nbhd(const Pm& p, const R (&v)[P][3][3], Nbhd<P, R>& n) {
+template <int P, class R>
+__device__ __forceinline__ void make_nbhd(const DevParams<R>& p, const R (&v)[P][3][3], Nbhd<P, R>& n) {
 #pragma unroll
   for (int a = 0; a < P; a++) {
     bool nz = false;
@@ -508,8 +484,8 @@ __device__ __forceinline__ void make_nbhd(const Pm& p, const R (&v)[P][3][3], Nb
 // ---------------------------------------------------------------- delta-phi
 
 // dA/dphi_a  (function_A_00.h:4-24 isotropic; function_A_01.h:4-71 anisotropic)
-template <int P, class R, class Pm>
-__device__ __forceinline__ R dAdphi(const Pm& p, const Nbhd<P, R>& n, int a) {
+template <int P, class R>
+__device__ __forceinline__ R dAdphi(const DevParams<R>& p, const Nbhd<P, R>& n, int a) {
   if (!p.anisotropy) {
     R sum = R(0);
 #pragma unroll
@@ -559,8 +535,8 @@ struct FaceQ {
   R rd[2];     // R^-1 * da_c/dq
 };
 
-template <class R, class Pm>
-__device__ __forceinline__ void face_q(const Pm& p, int a, int b, R u0, R u1, R flux, FaceQ<R>& f) {
+template <class R>
+__device__ __forceinline__ void face_q(const DevParams<R>& p, int a, int b, R u0, R u1, R flux, FaceQ<R>& f) {
   R u[2] = {u0, u1}, q[2], d[2];
   rot2(p.rot[a][b], u, q);
   f.flux = flux;
@@ -572,8 +548,8 @@ __device__ __forceinline__ void face_q(const Pm& p, int a, int b, R u0, R u1, R 
 }
 
 // div (dA / d grad phi_a)  (function_A_00.h:25-58 isotropic; function_A_01.h:101-219 anisotropic)
-template <int P, class R, class Pm>
-__device__ __forceinline__ R divdAdgradphi(const Pm& p, const Nbhd<P, R>& n, int a) {
+template <int P, class R>
+__device__ __forceinline__ R divdAdgradphi(const DevParams<R>& p, const Nbhd<P, R>& n, int a) {
   if (!p.anisotropy) {
     R sum = R(0);
 #pragma unroll
@@ -632,8 +608,8 @@ __device__ __forceinline__ R divdAdgradphi(const Pm& p, const Nbhd<P, R>& n, int
 // only in the sign of a zero, which leaves nonzero sums unchanged; the results
 // are returned as dA = 2(s1+s2) (entering lam as -dA + dG, where either zero
 // gives +0) and dG = 2(s1+s2) + 0 (zero normalised as in divdAdgradphi).
-template <int P, class R, class Pm>
-__device__ __forceinline__ void aniso_pairs(const Pm& p, const Nbhd<P, R>& n, const bool* want, R* dA,
+template <int P, class R>
+__device__ __forceinline__ void aniso_pairs(const DevParams<R>& p, const Nbhd<P, R>& n, const bool* want, R* dA,
                                             R* dG) {
   R a1[P], a2[P], g1[P], g2[P];
 #pragma unroll
@@ -723,8 +699,8 @@ __device__ __forceinline__ void aniso_pairs(const Pm& p, const Nbhd<P, R>& n, co
 }
 
 // dw/dphi_a  (functionW_01.h:6-39 obstacle, functionW_02.h:4-33 well)
-template <int P, class R, class Pm>
-__device__ __forceinline__ R dwdphi(const Pm& p, const R* ph, const bool* act, int a) {
+template <int P, class R>
+__device__ __forceinline__ R dwdphi(const DevParams<R>& p, const R* ph, const bool* act, int a) {
   R sum = R(0);
   if (p.obstacle) {
 #pragma unroll
@@ -797,8 +773,8 @@ __device__ __forceinline__ void project_simplex(const R* ph, const bool* act, R*
 
 // Active phases of a cell: |div phi_a| > 0 (calculate_divergence_phasefield.h:9-16).
 // Returns whether any phase is active.
-template <int P, class R, class Pm>
-__device__ __forceinline__ bool cell_active(const Pm& p, const Nbhd<P, R>& n, bool* act) {
+template <int P, class R>
+__device__ __forceinline__ bool cell_active(const DevParams<R>& p, const Nbhd<P, R>& n, bool* act) {
   bool any = false;
 #pragma unroll
   for (int a = 0; a < P; a++) {
@@ -819,8 +795,8 @@ __device__ __forceinline__ bool cell_active(const Pm& p, const Nbhd<P, R>& n, bo
 // dpsi / V under GP_MPI_DPSI_V, and mnz (4 Amp drand48() of the cell) adds
 // mnz phi_a (1 - phi_a) dpsi / V under p.mpi_noise
 // (MPI calculate_divergence_phasefield.h:335-343).
-template <int P, int C, class R, bool NI = false, bool MPI = false, class Pm>
-__device__ __forceinline__ void cell_dphi_rest(const Pm& p, const Nbhd<P, R>& n, const R* mu,
+template <int P, int C, class R, bool NI = false, bool MPI = false>
+__device__ __forceinline__ void cell_dphi_rest(const DevParams<R>& p, const Nbhd<P, R>& n, const R* mu,
                                                const bool* act, bool any, bool pairs, R* dA, R* dG, R* dp,
                                                R T = R(0), const uint32_t* nzw = nullptr, R amp = R(0),
                                                R mnz = R(0)) {
@@ -866,8 +842,8 @@ __device__ __forceinline__ void cell_dphi_rest(const Pm& p, const Nbhd<P, R>& n,
 
 // delta-phi of one cell  (calculate_divergence_phasefield.h:4-62)
 // (T: the cell's temperature, used with NI only)
-template <int P, int C, class R, bool NI = false, bool MPI = false, class Pm>
-__device__ __forceinline__ void cell_dphi(const Pm& p, const Nbhd<P, R>& n, const R* mu, R* dp,
+template <int P, int C, class R, bool NI = false, bool MPI = false>
+__device__ __forceinline__ void cell_dphi(const DevParams<R>& p, const Nbhd<P, R>& n, const R* mu, R* dp,
                                           R T = R(0), const uint32_t* nzw = nullptr, R amp = R(0),
                                           R mnz = R(0)) {
   bool act[P];
@@ -889,8 +865,8 @@ __device__ __forceinline__ R s_phi(const R* ph, int a) {
 }
 
 // D_ij of one cell  (functionD.h:1-15)
-template <int P, int C, class R, class Pm>
-__device__ __forceinline__ void cell_D(const Pm& p, const R* ph, R (&D)[C][C]) {
+template <int P, int C, class R>
+__device__ __forceinline__ void cell_D(const DevParams<R>& p, const R* ph, R (&D)[C][C]) {
 #pragma unroll
   for (int i = 0; i < C; i++)
 #pragma unroll
@@ -909,8 +885,8 @@ __device__ __forceinline__ void cell_D(const Pm& p, const R* ph, R (&D)[C][C]) {
 // ct_p / ct_q: tangential centred gradients at p and q (the face's tangential
 // gradient is their mean), phase fields, potentials and delta-phi of both cells.
 // With NI, c(mu) of the two cells is taken at their temperatures T_p, T_q.
-template <int P, int C, class R, bool NI = false, class Pm>
-__device__ __forceinline__ void face_jat(const Pm& p, const R* g_p, const R* ct_p, const R* ct_q,
+template <int P, int C, class R, bool NI = false>
+__device__ __forceinline__ void face_jat(const DevParams<R>& p, const R* g_p, const R* ct_p, const R* ct_q,
                                          const R* ph_p, const R* ph_q, const R* mu_p, const R* mu_q,
                                          const R* dp_p, const R* dp_q, bool enabled, R* jat, R T_p = R(0),
                                          R T_q = R(0)) {
@@ -1174,8 +1150,8 @@ __device__ __forceinline__ void cell_update(const Pm& p, const R* ph, const R* m
 // sum2 = 0; function_A_00.h returns 2*sum), obstacle/well terms without sign
 // tests (functionW_01.h:41-63, functionW_02.h:35-58), unweighted projection
 // (simplex_projection.h:50-90).
-template <int P, class R, class Pm>
-__device__ __forceinline__ R dwdphi_smooth(const Pm& p, const R* ph, const bool* act, int a) {
+template <int P, class R>
+__device__ __forceinline__ R dwdphi_smooth(const DevParams<R>& p, const R* ph, const bool* act, int a) {
   R sum = R(0);
 #pragma unroll
   for (int b = 0; b < P; b++)
@@ -1220,8 +1196,8 @@ __device__ __forceinline__ void project_unweighted(const R* ph, const bool* act,
   }
 }
 
-template <int P, int C, class R, class Pm>
-__device__ __forceinline__ void cell_dphi_smooth(const Pm& p, const Nbhd<P, R>& n, R* dp) {
+template <int P, int C, class R>
+__device__ __forceinline__ void cell_dphi_smooth(const DevParams<R>& p, const Nbhd<P, R>& n, R* dp) {
   R divphi[P], lam[P];
   bool act[P];
 #pragma unroll
@@ -1271,8 +1247,8 @@ __device__ __forceinline__ void cell_dphi_smooth(const Pm& p, const Nbhd<P, R>& 
 
 // mu update of the smoothing sweep: diffusion alone, general LU inverse for any
 // solver flag, mu + delta_mu (calculate_divergence_concentration.h:154-253)
-template <int P, int C, class R, class Pm>
-__device__ __forceinline__ void cell_update_smooth(const Pm& p, const R* ph, const R* mu,
+template <int P, int C, class R>
+__device__ __forceinline__ void cell_update_smooth(const DevParams<R>& p, const R* ph, const R* mu,
                                                    const R (&Dmf)[C][C], const R (&Dmb)[C][C],
                                                    const R (&Dmr)[C][C], const R (&Dml)[C][C],
                                                    const R* gmf, const R* gmb, const R* gmr, const R* gml,

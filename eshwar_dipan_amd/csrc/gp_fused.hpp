@@ -250,33 +250,20 @@ __global__ void __launch_bounds__(256) GP_HEAVY k_fused(const DevParams<R>* __re
 // bulk branch of cell_update with those zeros -- bit-identical to conc_cell.
 // bulk_mu takes the cell's phase vector ph, writes mu (and the binary32 low
 // parts) and returns the new phase vector in pho (ph + 0, the same bits).
-// bulk_mu_v takes mu of the five-point stencil already loaded, and the phase
-// tables from q (p, or a view of it with the cell's phase alone).
+// bulk_mu_v takes mu of the five-point stencil and the mobility Dm that the five
+// cells share (they carry the same phi), and the phase tables from q (p, or a
+// view of the cell's phase alone).
 template <int P, int C, class R, bool NI = false, class Pm>
-__device__ __forceinline__ void bulk_mu_v(const DevParams<R>& p, const Pm& q, const R* ph, const R* mc, const R* mf, const R* mb,
-                                          const R* mr, const R* ml, const R* __restrict__ mulo, R* __restrict__ mu_o,
-                                          R* __restrict__ mulo_o, int x, int y, R T, R* pho,
-                                          const R* lo_pre = nullptr, const R (*dm_pre)[CM] = nullptr) {
+__device__ __forceinline__ void bulk_mu_v(const DevParams<R>& p, const Pm& q, const R* ph, const R (&Dm)[C][C],
+                                          const R* mc, const R* mf, const R* mb, const R* mr, const R* ml,
+                                          const R* __restrict__ mulo, R* __restrict__ mu_o, R* __restrict__ mulo_o,
+                                          int x, int y, R T, R* pho, const R* lo_pre = nullptr) {
   R zp[P], z[C];
 #pragma unroll
   for (int a = 0; a < P; a++) zp[a] = R(0);
 #pragma unroll
   for (int k = 0; k < C; k++) z[k] = R(0);
-  // the five cells carry the same phi, hence the same mobility
-  R Dm[C][C], gmf[C], gmb[C], gmr[C], gml[C];
-  if (dm_pre) {  // the table of the one-hot phase (DevParams::Dm_bulk), the same values
-#pragma unroll
-    for (int k = 0; k < C; k++)
-#pragma unroll
-      for (int l = 0; l < C; l++) Dm[k][l] = dm_pre[k][l];
-  } else {
-    R D[C][C];
-    cell_D<P, C>(q, ph, D);
-#pragma unroll
-    for (int k = 0; k < C; k++)
-#pragma unroll
-      for (int l = 0; l < C; l++) Dm[k][l] = (D[k][l] + D[k][l]) * R(0.5);
-  }
+  R gmf[C], gmb[C], gmr[C], gml[C];
 #pragma unroll
   for (int k = 0; k < C; k++) {
     gmf[k] = div_dx(mf[k] - mc[k], p);
@@ -315,7 +302,31 @@ __device__ __forceinline__ void bulk_mu(const DevParams<R>& p, const R* ph, cons
     mr[k] = mu[idx(p, k, x, y + 1)];
     ml[k] = mu[idx(p, k, x, y - 1)];
   }
-  bulk_mu_v<P, C, R, NI>(p, p, ph, mc, mf, mb, mr, ml, mulo, mu_o, mulo_o, x, y, T, pho);
+  R D[C][C], Dm[C][C];
+  cell_D<P, C>(p, ph, D);
+#pragma unroll
+  for (int k = 0; k < C; k++)
+#pragma unroll
+    for (int l = 0; l < C; l++) Dm[k][l] = (D[k][l] + D[k][l]) * R(0.5);
+  bulk_mu_v<P, C, R, NI>(p, p, ph, Dm, mc, mf, mb, mr, ml, mulo, mu_o, mulo_o, x, y, T, pho);
+}
+
+// bulk_mu_v of a cell at the exact one-hot vector of phase a: that phase's tables
+// alone, and its mobility from the table formed on the host (Dm_bulk, the same
+// values).
+template <int C, class R, bool NI = false>
+__device__ __forceinline__ void bulk_mu_onehot(const DevParams<R>& p, int a, const R* mc, const R* mf, const R* mb,
+                                               const R* mr, const R* ml, const R* __restrict__ mulo,
+                                               R* __restrict__ mu_o, R* __restrict__ mulo_o, int x, int y, R T,
+                                               const R* lo_pre = nullptr) {
+  const PhaseParams<R> q(p, a);
+  const R one[1] = {R(1.0)};
+  R Dm[C][C], pho[1];
+#pragma unroll
+  for (int k = 0; k < C; k++)
+#pragma unroll
+    for (int l = 0; l < C; l++) Dm[k][l] = p.Dm_bulk[a][k][l];
+  bulk_mu_v<1, C, R, NI>(p, q, one, Dm, mc, mf, mb, mr, ml, mulo, mu_o, mulo_o, x, y, T, pho, lo_pre);
 }
 
 template <int P, int C, class R, bool NI = false>
@@ -355,13 +366,10 @@ __global__ void __launch_bounds__(256) k_bulk(const Inst<R>* __restrict__ inst, 
     R *phi_o = g.phi[par ^ 1], *mu_o = g.mu[par ^ 1], *mulo_o = g.mulo[par ^ 1];
     const int f = flag_i[tile];
     const bool held = flag_o[tile] == f;
-    const int id[1] = {f};
-    const SubParams<R, 1> q(p, id);
     for (int i = threadIdx.x; i < TX * TY; i += 256) {
       const int x = x0 + i / TY, y = y0 + i % TY;
       if (x > p.mesh_x + 2 || y > p.mesh_y + 2) continue;
-      R mc[C], mf[C], mb[C], mr[C], ml[C], po[1];
-      const R one[1] = {R(1.0)};
+      R mc[C], mf[C], mb[C], mr[C], ml[C];
 #pragma unroll
       for (int k = 0; k < C; k++) {
         mc[k] = mu[idx(p, k, x, y)];
@@ -370,8 +378,7 @@ __global__ void __launch_bounds__(256) k_bulk(const Inst<R>* __restrict__ inst, 
         mr[k] = mu[idx(p, k, x, y + 1)];
         ml[k] = mu[idx(p, k, x, y - 1)];
       }
-      bulk_mu_v<1, C, R>(p, q, one, mc, mf, mb, mr, ml, mulo, mu_o, mulo_o, x, y, R(0), po, (const R*)nullptr,
-                         p.Dm_bulk[f]);
+      bulk_mu_onehot<C, R>(p, f, mc, mf, mb, mr, ml, mulo, mu_o, mulo_o, x, y, R(0));
       if (!held) {  // the same bits as ph + 0
 #pragma unroll
         for (int a = 0; a < P; a++)
@@ -1035,11 +1042,7 @@ struct LightMu {
     const R T = NI ? temp_row(p, tb, y, true, tsh) : R(0);
     // the bulk branch reads phase cc alone: one local phase (over all nine it
     // took 242 registers, or 552 B of scratch at six waves per SIMD; now 42)
-    const int id[1] = {cc};
-    const SubParams<R, 1> q(p, id);
-    const R one[1] = {R(1.0)};
-    R po[1];
-    bulk_mu_v<1, C, R, NI>(p, q, one, mc, mf, mb, mr, ml, mulo, mu_o, mulo_o, x, y, T, po, lo, p.Dm_bulk[cc]);
+    bulk_mu_onehot<C, R, NI>(p, cc, mc, mf, mb, mr, ml, mulo, mu_o, mulo_o, x, y, T, lo);
     if (oo != cc) {  // the same bits as ph + 0
 #pragma unroll
       for (int a = 0; a < P; a++)
