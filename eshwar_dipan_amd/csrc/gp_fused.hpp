@@ -52,8 +52,8 @@ __device__ __forceinline__ const Inst<R>& inst_of(const Inst<R>* __restrict__ in
   return inst[tinst ? tinst[tile] : 0];
 }
 
-// Bulk-tile flag of a cell: the phase a if phi is one-hot in a (phi_a == 1, all
-// others == 0), -1 otherwise; -2 marks "no cell" in reductions.
+// One-hot code of a cell on the split paths (4, 5): the phase a if phi is one-hot
+// in a (phi_a == 1, all others == 0 of either sign), -1 otherwise.
 template <int P, class R>
 __device__ __forceinline__ int onehot_phase(const R* ph) {
   int a1 = -1, nz = 0;
@@ -65,8 +65,9 @@ __device__ __forceinline__ int onehot_phase(const R* ph) {
   return nz == 0 ? a1 : -1;
 }
 
-// Exact one-hot code of a phase vector: a if ph is bit for bit the one-hot
-// vector of phase a (1 in a, +0 in every other phase), -1 otherwise.
+// Exact one-hot code of a phase vector (tile flags, the tile paths' cell codes and
+// the one-hot path): a if ph is bit for bit the one-hot vector of phase a (1 in a,
+// +0 in every other phase), -1 otherwise.
 template <int P, class R>
 __device__ __forceinline__ int onehot_bits(const R* ph) {
   int a1 = -1, n1 = 0;
@@ -83,6 +84,7 @@ __device__ __forceinline__ int onehot_bits(const R* ph) {
   return z && n1 == 1 ? a1 : -1;
 }
 
+// Tile flags: one phase for all cells, or -1; -2 marks "no cell" in reductions.
 __device__ __forceinline__ int flag_combine(int x, int y) { return x == -2 ? y : y == -2 ? x : (x == y ? x : -1); }
 
 // Block-wide combination of per-thread flags; result valid in thread 0.
@@ -348,8 +350,10 @@ __device__ __forceinline__ void bulk_cell(const DevParams<R>& p, const R* __rest
 // the cells and at their ghost images (flag_o describes the state of two steps
 // back until it is overwritten here; the sweeps that set it write both, k_flags
 // looks at both).
-// The sweep is bound by memory and now moves the mu planes alone: on 64 grids of
-// 64^2 to 512^2 (two phases, binary64) 143 -> 58 us a step, 100 MB at 1.7 TB/s.
+// The sweep moves the mu planes alone: on 64 grids of 64^2 to 512^2 (two phases,
+// binary64) 143 -> 58 us a step.  That is 100 MB at 1.7 TB/s, below half of a
+// large copy's rate; what bounds it is not known (reading the next tile's list
+// entry, grid and flags ahead of the current tile's update changed nothing).
 template <int P, int C, class R, int TX, int TY>
 __global__ void __launch_bounds__(256) k_bulk(const Inst<R>* __restrict__ inst, const int* __restrict__ tinst, int par,
                                               const int* __restrict__ list, const int* __restrict__ count,
@@ -1266,7 +1270,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(onehot
 // densely packed waves.
 //
 // The phase sweep also writes a one-byte code per cell: the phase a if phi is
-// one-hot in a and delta-phi is +0 in every phase, else -1.  A cell whose 3x3
+// the exact one-hot vector of a and delta-phi is +0 in every phase, else -1.  A cell whose 3x3
 // block carries one code a >= 0 meets the bulk_cell conditions.
 template <int P, int C, class R, int TX, int TY>
 __global__ void __launch_bounds__(256) GP_HEAVY k_phase_tiles(const Inst<R>* __restrict__ inst, const int* __restrict__ tinst,

@@ -42,9 +42,6 @@ namespace GPK_NS {
 // SIMD leave (the dense phase sweep spilled 2.5 KB per lane, the dense mu
 // sweep 0.6 KB): its dense sweeps run at one wave per SIMD (1.6x the merged
 // launch at two waves).  Binary32 spills 0.8 KB and is faster at two waves.
-// With passes by the phases a cell holds the launches are separate too: merged,
-// the light waves at six phases were held to the dense pass's two per SIMD (64
-// us at 1531 x 1021, against 42 + 21 us for the two launches).
 template <int P, class R>
 constexpr bool onehot_wide() { return P >= 9; }
 template <int P, class R>
@@ -174,8 +171,8 @@ __device__ __forceinline__ void phase_cell(const DevParams<R>& p, const R* __res
 // mu and phi update of interior cell (x,y) from its 3x3 phi block v, the mu of
 // its five-point stencil, its delta-phi and the antitrapping fluxes of its four
 // faces; writes the cell and its ghost images.  Kahan adds the mu increment to
-// mu + mulo (binary32).  Returns the one-hot phase of the updated phi (-1 if
-// not one-hot).
+// mu + mulo (binary32).  Returns the phase of which the updated phi is
+// the exact one-hot vector (-1 if none).
 template <int P, int C, class R, bool Kahan, bool NI = false>
 __device__ __forceinline__ int conc_apply(const DevParams<R>& p, const R (&v)[P][3][3], const R* mc, const R* mf,
                                           const R* mb, const R* mr, const R* ml, const R* dc, const R* jf,

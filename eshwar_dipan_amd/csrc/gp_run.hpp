@@ -384,7 +384,8 @@ int run_compact(gp_ctx *c, long nsteps) {
 // when the previous step was not a step of this path (c->oh_valid == 0), also
 // for nsteps == 0, so that a graph captured after such a call starts valid.
 // The segmented lists and their counters live in c->dcells6 (kSegInts
-// counters, then 256 cells per block of each light launch).
+// counters, then a slot for every cell of each light launch's blocks:
+// kPhaseCells per block of the phase sweep, kMuCells per block of the mu sweep).
 template <int P, int C, class R, bool NI>
 int run_onehot(gp_ctx *c, long nsteps) {
   if (c->rx > 65535 || c->ry > 65535) return GP_E_UNSUPPORTED;  // list entries pack x and y in 16 bits
